@@ -32,98 +32,13 @@
 #include <mutex>
 
 #include "common.h"
+#include "gemm_big.h"
+#include "gemm_epi.h"
 
 namespace {
 
 constexpr int BK = 64;
 
-// Tile order. Dispatch sends workgroup b to XCD (b % 8), so each XCD is given a contiguous run of the tile sequence
-// (split-major, then tile). Inside a run, tiles go in groups of GM row panels, column-major within a group: the 32
-// workgroups an XCD runs at once then share GM panels of A and a few panels of W in that XCD's L2, instead of
-// sweeping every row panel of A past one W panel. Grids with at most GM row panels keep plain column-major order.
-// GM = 8, and 4 for the 192- and 256-row tiles of large grids (1-3 % faster there than 8; 16 and 32 were slower).
-template <int GM = 8>
-__device__ __forceinline__ void tile_of(int b, int tiles_m, int tiles_n, int splits, int& tm, int& tn, int& split) {
-  const int nt = tiles_m * tiles_n, ntot = nt * splits;
-  const int per = ntot / 8, rem = ntot % 8, xcd = b % 8, idx = b / 8;
-  const int t = (xcd < rem) ? xcd * (per + 1) + idx : rem * (per + 1) + (xcd - rem) * per + idx;
-  const int tile = t % nt;
-  split = t / nt;
-  const int grp = tile / (GM * tiles_n), first = grp * GM, gs = min(tiles_m - first, GM);
-  const int r = tile - grp * GM * tiles_n;
-  tm = first + r % gs;
-  tn = r / gs;
-}
-
-// Epilogue of one 4-column group (output row m, columns n .. n+3) from fp32 sums s: + bias, round to bf16, activation
-// ACT (1 GELU-tanh, 2 GELU-erf; rounded again; skipped for columns >= act_ncols when act_ncols > 0), + residual
-// (fp32 add, rounded once more). ACT 3 is the gated GELU of interleaved (gate, up) column pairs, written to columns
-// n / 2, n / 2 + 1.
-template <int V>
-struct IntC {
-  static constexpr int value = V;
-};
-// I8: s holds int32 accumulator bits; the linear output is ((float)acc * sa) * sw + bias in fp32 and any GELU applies
-// to that fp32 value before the one bf16 rounding (the W8A8 epilogue); a residual is then added to the rounded value.
-// HR: 0 / 1 = no residual / a residual, known at compile time; 2 = has_r decides. The activation is computed for every
-// column and then selected (act_ncols varies across the lanes of a wave: a branch per group would serialise the
-// exp / rcp chains of the groups instead of interleaving them).
-template <int ACT, bool I8 = false, int HR = 2>
-__device__ __forceinline__ u32x2 epi_val(const f32x4& s, const f32x4& bv, const u32x2& rv, bool has_r, int n,
-                                         int act_ncols, float sa = 0.f, const f32x4& sw = f32x4{0.f, 0.f, 0.f, 0.f}) {
-  const bool hr = HR == 2 ? has_r : HR == 1;
-  float v[4];
-  if constexpr (I8) {
-    static_assert(ACT != 3, "no gated GELU in the int8 path");
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-      const float t = (float)__float_as_int(s[e]) * sa;
-      v[e] = t * sw[e] + bv[e];
-    }
-    if constexpr (ACT == 1 || ACT == 2) {
-      const bool on = act_ncols <= 0 || n < act_ncols;
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        const float g = ACT == 1 ? gelu_tanh(v[e]) : gelu_erf(v[e]);
-        v[e] = on ? g : v[e];
-      }
-    }
-    if (hr) {
-      v[0] = rbf(v[0]) + lo_bf(rv.x);
-      v[1] = rbf(v[1]) + hi_bf(rv.x);
-      v[2] = rbf(v[2]) + lo_bf(rv.y);
-      v[3] = rbf(v[3]) + hi_bf(rv.y);
-    }
-    return u32x2{pack2(v[0], v[1]), pack2(v[2], v[3])};
-  }
-#pragma unroll
-  for (int e = 0; e < 4; e++) v[e] = rbf(s[e] + bv[e]);
-  u32x2 o;
-  if constexpr (ACT == 3) {
-    o.x = pack2(rbf(gelu_tanh(v[0])) * v[1], rbf(gelu_tanh(v[2])) * v[3]);
-    o.y = 0;
-  } else {
-    if constexpr (ACT == 1 || ACT == 2) {
-      // the activation's bf16 rounding: explicit before a residual add, else the final pack's own rounding
-      const bool on = act_ncols <= 0 || n < act_ncols;
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        float g = ACT == 1 ? gelu_tanh(v[e]) : gelu_erf(v[e]);
-        if (hr) g = rbf(g);
-        v[e] = on ? g : v[e];
-      }
-    }
-    if (hr) {
-      v[0] += lo_bf(rv.x);
-      v[1] += hi_bf(rv.x);
-      v[2] += lo_bf(rv.y);
-      v[3] += hi_bf(rv.y);
-    }
-    o.x = pack2(v[0], v[1]);
-    o.y = pack2(v[2], v[3]);
-  }
-  return o;
-}
 // Group result into the LDS staging tile (row pitch SP elements) at tile row r, tile column c (ACT 3: column c / 2).
 template <int ACT, int SP>
 __device__ __forceinline__ void stage_val(uint16_t* st, int r, int c, const u32x2& o) {
@@ -171,17 +86,6 @@ __device__ __forceinline__ u32x2 res4(const uint16_t* __restrict__ R, long ldr, 
   if (r_rows > 0) rm %= r_rows;
   return *reinterpret_cast<const u32x2*>(R + (long)rm * ldr + min(n, N - 4));
 }
-// Run f(IntC<act>) for the runtime activation code act (0..3).
-template <typename F>
-__device__ __forceinline__ void with_act(int act, F&& f) {
-  switch (act) {
-    case 1: f(IntC<1>{}); break;
-    case 2: f(IntC<2>{}); break;
-    case 3: f(IntC<3>{}); break;
-    default: f(IntC<0>{}); break;
-  }
-}
-
 // Scheduling groups for one substep of the software pipeline: R LDS reads (of the next substep's fragments), each
 // followed by its share of the F MFMAs (of this substep), so the reads are spread under the matrix work.
 template <int R, int F, int r = 0>
@@ -1063,6 +967,7 @@ constexpr Cfg kCfgs[] = {{128, 128, 4, 1, 0, 4}, {64, 128, 4, 1, 0, 4}, {128, 64
                          {64, 64, 4, 2, 1, 4},   {64, 128, 4, 1, 1, 4},  {128, 64, 4, 1, 1, 4}, {64, 64, 3, 3, 1, 4},
                          {64, 96, 2, 3, 1, 4},   {64, 64, 6, 1, 1, 4},   {96, 64, 2, 3, 1, 4},
                          // 8-wave tiles for large grids: 2 waves per SIMD hide each other's LDS reads and barriers
+                         // (256 x 256 is gemm_big.hip's persistent tile in bf16, an 8-wave tile in int8)
                          {256, 256, 2, 1, 0, 8}, {256, 128, 3, 1, 0, 8}, {128, 256, 3, 1, 0, 8},
                          // 4 waves of 128 x 128: 8 LDS reads per 16 MFMAs (LDS traffic at 3/4 of the MFMA time)
                          {256, 256, 2, 1, 0, 4},
@@ -1074,7 +979,7 @@ constexpr Cfg kCfgs[] = {{128, 128, 4, 1, 0, 4}, {64, 128, 4, 1, 0, 4}, {128, 64
                          // (8 row tiles, the same 768 padded rows as 128 and a third more workgroups)
                          {96, 128, 4, 1, 0, 4},
                          // large grids whose N is a multiple of 192 (1152, 3456): 192 x 192 over two k groups with a
-                         // 3-stage ring (two stages in flight), and 256 x 192 on 4 x 2 waves
+                         // 3-stage ring (two stages in flight), and gemm_big.hip's persistent 256 x 192 tile
                          {192, 192, 3, 1, 0, 8, 2}, {256, 192, 2, 1, 0, 8},
                          // 730-row prompt-prefix GEMMs: 4 row tiles of 192 x 64 column tiles of 128 = 256 workgroups
                          // for N = 8192; two k groups of 2 x 2 waves, 4-stage ring
@@ -1322,11 +1227,16 @@ extern "C" int mx_gemm_bf16(hipStream_t st, int cfg, int splits, const uint16_t*
     case 6: e = L_(64, 64, 3); break;
     case 7: e = L_(128, 128, 2); break;
     case 23: e = launch<96, 128, 1, 4, 4>(st, splits, A, lda, W, ldw, bias, R, ldr, r_rows, C, ldc, M, N, K, Kw, act, act_ncols, ws, cnt); break;
-    case 15: e = launch<256, 256, 2, 4, 2>(st, splits, A, lda, W, ldw, bias, R, ldr, r_rows, C, ldc, M, N, K, Kw, act, act_ncols, ws, cnt); break;
+    case 15: case 25: {
+      // the persistent tiles; what they do not take (rows of C or R not in whole 16-byte chunks, K <= 192) runs on the
+      // 128 x 128 tile of config 7: the same bits
+      const BigGemm g{A, lda, W, ldw, bias, R, ldr, r_rows, C, ldc, M, N, K, Kw, act_ncols};
+      e = gemm_big_fits(act, g) ? launch_gemm_big(st, kCfgs[cfg].bn, act, g) : L_(128, 128, 2);
+      break;
+    }
     case 16: e = launch<256, 128, 4, 2, 3>(st, splits, A, lda, W, ldw, bias, R, ldr, r_rows, C, ldc, M, N, K, Kw, act, act_ncols, ws, cnt); break;
     case 17: e = launch<128, 256, 2, 4, 3>(st, splits, A, lda, W, ldw, bias, R, ldr, r_rows, C, ldc, M, N, K, Kw, act, act_ncols, ws, cnt); break;
     case 18: e = L_(256, 256, 2); break;
-    case 25: e = launch<256, 192, 4, 2, 2>(st, splits, A, lda, W, ldw, bias, R, ldr, r_rows, C, ldc, M, N, K, Kw, act, act_ncols, ws, cnt); break;
 #define H_(BM, BN, S) launch_kh2<BM, BN, S>(st, splits, A, lda, W, ldw, bias, R, ldr, r_rows, C, ldc, M, N, K, Kw, act, act_ncols)
     case 19: e = H_(128, 128, 4); break;
     case 20: e = H_(64, 128, 4); break;
