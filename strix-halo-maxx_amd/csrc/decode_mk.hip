@@ -131,6 +131,7 @@ __device__ __forceinline__ int b_quarter(int j) { return 2 * (j / (JB / 2)) + (j
 __device__ __forceinline__ int rot_wave(int wg, int wave, int k) { return ((wg & ~7) + ((wg + ROT * k) & 7)) * GW + wave; }
 constexpr int MK_ROUNDS = 16;                               // key rounds of 8 keys per compute wave: 1024 keys
 constexpr int MK_MAXKEYS = MK_ROUNDS * 8 * MK_W;
+constexpr int MK_LONGKEYS = 2048;                           // the LONG form: passes of MK_MAXKEYS keys
 constexpr int MK_MAXL = 32;                                 // layers the LDS copy of the layer table holds
 constexpr int MK_LP = 13;                                   // pointers per layer descriptor
 
@@ -447,7 +448,7 @@ __device__ __forceinline__ void static_for(F&& f) {
 
 typedef u32x4 Buf[8];  // one unit in flight: 2 rows x 4 chunks, a half fc2 row (8 chunks) or a proj row (4)
 
-template <bool I8>
+template <bool I8, bool LONG>
 __global__ __launch_bounds__(MK_T) void decode_mk_kernel(MkArgs a) {
   using RC = RingCfg<I8>;
   constexpr int SA = RC::SA, B0 = RC::B0, B1 = RC::B1, BH = RC::BH, NSLOT = RC::NSLOT;
@@ -594,7 +595,11 @@ __global__ __launch_bounds__(MK_T) void decode_mk_kernel(MkArgs a) {
       // key at byte 128 key), issued before the exchange wave's wait for q / k / v; lane l of wave w takes key
       // w * 8 + (l >> 3) + 64 r in round r, dims 8 (l & 7) .. + 7. The buffer range of both caches ends at row pos, so
       // rows at and past pos read as zeros (masked below; the new token's own key is scored by wave 0 from LDS).
-      // One-pass softmax per wave, merged by the exchange wave.
+      // One-pass softmax per wave, merged by the exchange wave. LONG: keys past the first 1024 follow in passes of
+      // 1024 through the same registers and LDS rows (a wave reads only the rows it copied itself, so it refills them
+      // without a barrier), K while the pass before it is weighted, V after it; the wave's maximum, sum and output are
+      // rescaled from pass to pass. The second pass's V copy is waited for, about 3 us a layer: 4 W8A8 layers and the LM
+      // head take 114 us at 1000 keys, 127 at 1025, 128 at 1500, 131 at 2000; the per-layer kernels 132 / 136 / 147 / 148.
       const int sub = lane & 7, kg = lane >> 3;
       const uint32_t koff = (uint32_t)(wave * 8 + kg) * 128u + (uint32_t)sub * 16u;
       for (int l = 0; l < NL; l++) {
@@ -615,55 +620,78 @@ __global__ __launch_bounds__(MK_T) void decode_mk_kernel(MkArgs a) {
         bar();  // q, k, v ready
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's K registers and V rows have landed
         const u32x4 qp = *reinterpret_cast<const u32x4*>(&qr[sub * 8]);
-        float sv[MK_ROUNDS];
-        float mb = -INFINITY;
+        float m = -1e30f, lsum = 0.f, o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        for (int k0 = 0;; k0 += MK_MAXKEYS) {
+          const bool more = LONG && k0 + MK_MAXKEYS < pos;
+          float sv[MK_ROUNDS];
+          float mb = -INFINITY;
 #pragma unroll
-        for (int r = 0; r < MK_ROUNDS; r++) {
-          const int key = wave * 8 + kg + 64 * r;
-          float sc = dot8d(kk[r], qp, 0.f);
-          sc += __shfl_xor(sc, 1, 64);
-          sc += __shfl_xor(sc, 2, 64);
-          sc += __shfl_xor(sc, 4, 64);
-          sc = key < pos ? sc * a.scale_log2 : -INFINITY;
-          sv[r] = sc;
-          mb = fmaxf(mb, sc);
-        }
-        float snew = -INFINITY;  // the new token's key, wave 0
-        if (wave == 0) {
-          float sc = dot8d(*reinterpret_cast<const u32x4*>(&kr[sub * 8]), qp, 0.f);
-          sc += __shfl_xor(sc, 1, 64);
-          sc += __shfl_xor(sc, 2, 64);
-          sc += __shfl_xor(sc, 4, 64);
-          snew = sc * a.scale_log2;
-          mb = fmaxf(mb, snew);
-        }
-        const float m = fmaxf(wave_max(mb), -1e30f);  // a wave with no key in range: p = 0, not NaN
-        float lsum = 0.f, o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int r = 0; r < MK_ROUNDS; r++) {
-          // rows past the range: p = 0, and the LDS row is zeroed here whatever the copy left in it (0 x NaN = NaN)
-          const u32x4 zero4 = {0u, 0u, 0u, 0u};
-          const u32x4 vl = *reinterpret_cast<const u32x4*>(big + (wave * 8 + kg + 64 * r) * 128 + sub * 16);
-          const u32x4 vv = wave * 8 + kg + 64 * r < pos ? vl : zero4;
-          const float pr = rbf(__builtin_amdgcn_exp2f(sv[r] - m));
-          if (sub == 0) lsum += pr;
-#pragma unroll
-          for (int e = 0; e < 4; e++) {
-            const uint32_t ve = vv[e];
-            o[2 * e] = __builtin_fmaf(pr, lo_bf(ve), o[2 * e]);
-            o[2 * e + 1] = __builtin_fmaf(pr, hi_bf(ve), o[2 * e + 1]);
+          for (int r = 0; r < MK_ROUNDS; r++) {
+            const int key = k0 + wave * 8 + kg + 64 * r;
+            float sc = dot8d(kk[r], qp, 0.f);
+            sc += __shfl_xor(sc, 1, 64);
+            sc += __shfl_xor(sc, 2, 64);
+            sc += __shfl_xor(sc, 4, 64);
+            sc = key < pos ? sc * a.scale_log2 : -INFINITY;
+            sv[r] = sc;
+            mb = fmaxf(mb, sc);
           }
-        }
-        if (wave == 0 && kg == 0) {
-          const u32x4 vv = *reinterpret_cast<const u32x4*>(&qkvh[2 * MK_HD + sub * 8]);
-          const float pr = rbf(__builtin_amdgcn_exp2f(snew - m));
-          if (sub == 0) lsum += pr;
+          const uint32_t ko2 = ko + (uint32_t)(k0 + MK_MAXKEYS) * 128u;
+          if (more) {
 #pragma unroll
-          for (int e = 0; e < 4; e++) {
-            const uint32_t ve = vv[e];
-            o[2 * e] = __builtin_fmaf(pr, lo_bf(ve), o[2 * e]);
-            o[2 * e + 1] = __builtin_fmaf(pr, hi_bf(ve), o[2 * e + 1]);
+            for (int r = 0; r < MK_ROUNDS; r++) kk[r] = __builtin_amdgcn_raw_buffer_load_b128(rk, ko2 + 8192u * r, 0, 0);
           }
+          const bool first = !LONG || k0 == 0;
+          float snew = -INFINITY;  // the new token's key, wave 0
+          if (wave == 0 && first) {
+            float sc = dot8d(*reinterpret_cast<const u32x4*>(&kr[sub * 8]), qp, 0.f);
+            sc += __shfl_xor(sc, 1, 64);
+            sc += __shfl_xor(sc, 2, 64);
+            sc += __shfl_xor(sc, 4, 64);
+            snew = sc * a.scale_log2;
+            mb = fmaxf(mb, snew);
+          }
+          const float mn = fmaxf(wave_max(mb), m);  // a wave with no key in range: p = 0, not NaN
+          if (!first) {
+            const float f = __builtin_amdgcn_exp2f(m - mn);
+            lsum *= f;
+#pragma unroll
+            for (int e = 0; e < 8; e++) o[e] *= f;
+          }
+          m = mn;
+#pragma unroll
+          for (int r = 0; r < MK_ROUNDS; r++) {
+            // rows past the range: p = 0, and the LDS row is zeroed here whatever the copy left in it (0 x NaN = NaN)
+            const u32x4 zero4 = {0u, 0u, 0u, 0u};
+            const u32x4 vl = *reinterpret_cast<const u32x4*>(big + (wave * 8 + kg + 64 * r) * 128 + sub * 16);
+            const u32x4 vv = k0 + wave * 8 + kg + 64 * r < pos ? vl : zero4;
+            const float pr = rbf(__builtin_amdgcn_exp2f(sv[r] - m));
+            if (sub == 0) lsum += pr;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+              const uint32_t ve = vv[e];
+              o[2 * e] = __builtin_fmaf(pr, lo_bf(ve), o[2 * e]);
+              o[2 * e + 1] = __builtin_fmaf(pr, hi_bf(ve), o[2 * e + 1]);
+            }
+          }
+          if (wave == 0 && kg == 0 && first) {
+            const u32x4 vv = *reinterpret_cast<const u32x4*>(&qkvh[2 * MK_HD + sub * 8]);
+            const float pr = rbf(__builtin_amdgcn_exp2f(snew - m));
+            if (sub == 0) lsum += pr;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+              const uint32_t ve = vv[e];
+              o[2 * e] = __builtin_fmaf(pr, lo_bf(ve), o[2 * e]);
+              o[2 * e + 1] = __builtin_fmaf(pr, hi_bf(ve), o[2 * e + 1]);
+            }
+          }
+          if (!more) break;
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's V rows are read
+#pragma unroll
+          for (int r = 0; r < MK_ROUNDS; r++)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                rv, (__attribute__((address_space(3))) void*)(big + (wave * 8 + 64 * r) * 128), 16, ko2 + 8192u * r, 0, 0, 0);
+          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         }
 #pragma unroll
         for (int e = 0; e < 8; e++) {
@@ -699,7 +727,9 @@ __global__ __launch_bounds__(MK_T) void decode_mk_kernel(MkArgs a) {
         }
         if constexpr (I8) {
           bar();  // g gathered
-          quant_block_i8<MK_F / 8>(gs, gq, qred, tid);
+          int tq = tid;
+          if (LONG) asm volatile("" : "+v"(tq));  // its LDS addresses stay in the layer's loop: hoisted, one spills
+          quant_block_i8<MK_F / 8>(gs, gq, qred, tq);
 #pragma unroll
           for (int j = 0; j < NU; j++) {  // half j of the row
             int acc = 0;
@@ -1146,14 +1176,15 @@ extern "C" int mx_decode_mk_words(void) { return LL_WORDS; }
 extern "C" int mx_decode_mk_grid(void) { return MK_G; }
 
 namespace {
-template <bool I8>
+template <bool I8, bool LONG>
 int launch_mk(hipStream_t st, const void* layers, int nl, int ctx, const uint16_t* lnf_g, const uint16_t* lnf_b,
               const uint16_t* wlm, const float* blm, int V, const uint16_t* wte, const float* cs, float eps, float scale,
               uint16_t* x, int* state, int pos_base, int* tokens, int cap, uint16_t* logits, uint64_t* ll,
               uint32_t* ep) {
   if (!layers || !lnf_g || !lnf_b || !wlm || !blm || !wte || !cs || !x || !state || !tokens || !ll || !ep)
     return MX_ENULL;
-  if (nl < 1 || nl > MK_MAXL || ctx < 1 || ctx > MK_MAXKEYS || V < 1 || V > 65536 || cap < 1 || pos_base < 0)
+  if (nl < 1 || nl > MK_MAXL || ctx < 1 || ctx > (LONG ? MK_LONGKEYS : MK_MAXKEYS) || V < 1 || V > 65536 || cap < 1 ||
+      pos_base < 0)
     return MX_ESHAPE;
   if (((uintptr_t)x | (uintptr_t)wlm | (uintptr_t)wte) & 15) return MX_ELAYOUT;
   int dev = 0, ncu = 0;
@@ -1167,7 +1198,7 @@ int launch_mk(hipStream_t st, const void* layers, int nl, int ctx, const uint16_
   a.eps = eps, a.scale_log2 = scale * 1.4426950408889634f;
   a.lnf_g = lnf_g, a.lnf_b = lnf_b, a.wlm = wlm, a.blm = blm, a.wte = wte, a.cs = cs;
   a.x = x, a.state = state, a.tokens = tokens, a.logits = logits, a.ll = ll, a.ep = ep;
-  hipLaunchKernelGGL(decode_mk_kernel<I8>, dim3(MK_G), dim3(MK_T), 0, st, a);
+  hipLaunchKernelGGL((decode_mk_kernel<I8, LONG>), dim3(MK_G), dim3(MK_T), 0, st, a);
   return hipGetLastError() == hipSuccess ? MX_OK : MX_ELAUNCH;
 }
 }  // namespace
@@ -1181,8 +1212,8 @@ extern "C" int mx_decode_step_mk(hipStream_t st, const void* layers, int nl, int
                                  const uint16_t* lnf_b, const uint16_t* wlm, const float* blm, int V,
                                  const uint16_t* wte, const float* cs, float eps, float scale, uint16_t* x, int* state,
                                  int pos_base, int* tokens, int cap, uint16_t* logits, uint64_t* ll, uint32_t* ep) {
-  return launch_mk<false>(st, layers, nl, ctx, lnf_g, lnf_b, wlm, blm, V, wte, cs, eps, scale, x, state, pos_base,
-                          tokens, cap, logits, ll, ep);
+  return launch_mk<false, false>(st, layers, nl, ctx, lnf_g, lnf_b, wlm, blm, V, wte, cs, eps, scale, x, state,
+                                 pos_base, tokens, cap, logits, ll, ep);
 }
 
 // The same step with the W8A8 text Linears: each descriptor's wqf / w2 / wp are int8 (the same shapes, one byte per
@@ -1192,8 +1223,27 @@ extern "C" int mx_decode_step_mk_i8(hipStream_t st, const void* layers, int nl, 
                                     const uint16_t* wte, const float* cs, float eps, float scale, uint16_t* x,
                                     int* state, int pos_base, int* tokens, int cap, uint16_t* logits, uint64_t* ll,
                                     uint32_t* ep) {
-  return launch_mk<true>(st, layers, nl, ctx, lnf_g, lnf_b, wlm, blm, V, wte, cs, eps, scale, x, state, pos_base,
-                         tokens, cap, logits, ll, ep);
+  return launch_mk<true, false>(st, layers, nl, ctx, lnf_g, lnf_b, wlm, blm, V, wte, cs, eps, scale, x, state,
+                                pos_base, tokens, cap, logits, ll, ep);
+}
+
+// The same steps for caches of up to 2048 positions (the model's whole context): the attention takes the keys past the
+// first 1024 in a second pass. Kernels of their own: the one-pass form keeps its code.
+extern "C" int mx_decode_step_mk_long(hipStream_t st, const void* layers, int nl, int ctx, const uint16_t* lnf_g,
+                                      const uint16_t* lnf_b, const uint16_t* wlm, const float* blm, int V,
+                                      const uint16_t* wte, const float* cs, float eps, float scale, uint16_t* x,
+                                      int* state, int pos_base, int* tokens, int cap, uint16_t* logits, uint64_t* ll,
+                                      uint32_t* ep) {
+  return launch_mk<false, true>(st, layers, nl, ctx, lnf_g, lnf_b, wlm, blm, V, wte, cs, eps, scale, x, state,
+                                pos_base, tokens, cap, logits, ll, ep);
+}
+extern "C" int mx_decode_step_mk_long_i8(hipStream_t st, const void* layers, int nl, int ctx, const uint16_t* lnf_g,
+                                         const uint16_t* lnf_b, const uint16_t* wlm, const float* blm, int V,
+                                         const uint16_t* wte, const float* cs, float eps, float scale, uint16_t* x,
+                                         int* state, int pos_base, int* tokens, int cap, uint16_t* logits,
+                                         uint64_t* ll, uint32_t* ep) {
+  return launch_mk<true, true>(st, layers, nl, ctx, lnf_g, lnf_b, wlm, blm, V, wte, cs, eps, scale, x, state,
+                               pos_base, tokens, cap, logits, ll, ep);
 }
 
 // Bytes of one layer descriptor in the layers array of mx_decode_step_mk(_i8): 13 device pointers (ln_g, ln_b, wqf,

@@ -126,12 +126,12 @@ class TextDecoder:
         self.steps = 0
         self.graph = None
         # one launch per decode step (mx_decode_step_mk, or mx_decode_step_mk_i8 for the W8A8 Linears) where its
-        # shapes hold: the 2048-wide, 32 x 64-head, 8192-MLP model, a cache of at most 1024 positions, one attention
-        # split, and a device with a CU for each of its workgroups; the per-layer kernels above otherwise (use_mk =
-        # False selects them too)
+        # shapes hold: the 2048-wide, 32 x 64-head, 8192-MLP model, a cache of at most 2048 positions (past 1024 its
+        # _long form, whose attention takes the keys in two passes), one attention split, and a device with a CU for
+        # each of its workgroups; the per-layer kernels above otherwise (use_mk = False selects them too)
         self.mk_layers = self.mk_ll = self.mk_ep = None
         if (dev.type == "cuda" and attn_splits == 1 and (self.D, self.H, self.hd, c["ff"]) == (2048, 32, 64, 8192)
-                and ctx <= 1024 and self.V <= 65536
+                and ctx <= 2048 and self.V <= 65536
                 and torch.cuda.get_device_properties(dev).multi_processor_count >= lib.mx_decode_mk_grid()):
             self._init_mk()
         self.use_mk = self.mk_layers is not None
@@ -390,14 +390,14 @@ class TextDecoder:
         lib = _lib.load()
         if self.use_mk:
             cap = max(1, min(self.ctx - self.pos_base + 1, self.ctx))
-            fn = lib.mx_decode_step_mk_i8 if self.w8a8 else lib.mx_decode_step_mk
+            fn = getattr(lib, "mx_decode_step_mk" + ("_long" if self.ctx > 1024 else "") + ("_i8" if self.w8a8 else ""))
             _lib.check(fn(st, self.mk_layers.data_ptr(), len(self.blocks), self.ctx,
-                                             self.post_ln[0].data_ptr(), self.post_ln[1].data_ptr(),
-                                             self.w_lm.data_ptr(), self.b_lm.data_ptr(), self.V, self.wte.data_ptr(),
-                                             self.cs.data_ptr(), float(self.eps), float(self.hd ** -0.5),
-                                             self.xd[0].data_ptr(), self.state.data_ptr(), self.pos_base,
-                                             self.tokens.data_ptr(), cap, ptr(self.logits) if logits else None,
-                                             self.mk_ll.data_ptr(), self.mk_ep.data_ptr()), "mx_decode_step_mk")
+                          self.post_ln[0].data_ptr(), self.post_ln[1].data_ptr(),
+                          self.w_lm.data_ptr(), self.b_lm.data_ptr(), self.V, self.wte.data_ptr(),
+                          self.cs.data_ptr(), float(self.eps), float(self.hd ** -0.5),
+                          self.xd[0].data_ptr(), self.state.data_ptr(), self.pos_base,
+                          self.tokens.data_ptr(), cap, ptr(self.logits) if logits else None,
+                          self.mk_ll.data_ptr(), self.mk_ep.data_ptr()), "mx_decode_step_mk")
             return
         xi = 0
         for i, b in enumerate(self.blocks):

@@ -477,6 +477,32 @@ def test_decode_reaches_the_last_cache_row(dev):
     assert len(neither) == 0 and dec.mk_error() == 0 and dec.mk_fallbacks == 0
 
 
+@pytest.mark.parametrize("w8a8", [False, True])
+@pytest.mark.parametrize("start", [1022, 1535, 2042])
+def test_one_launch_step_past_1024_keys(dev, start, w8a8):
+    """The _long one-launch step (ctx 2048) against the per-layer kernels, 6 greedy steps from position start: across
+    the edge of its first pass of 1024 keys, inside the second pass (1535 .. 1540: whole rounds of 64 keys end), and
+    up to the last cache row (2047). Tolerances as for the one-pass form: the two differ by fp32 summation orders
+    (5e-3), or by an int8 step of the LayerNorm's output (2e-2)."""
+    dec = mt.TextDecoder(S.text_weights(2, layers=2), ctx=2048, w8a8=w8a8)
+    assert dec.use_mk
+    img = S.activations(7, (729, 2048), "img").to(dev)
+    prompt = S.prompt_ids(8, start - 730)
+    out = {}
+    for mk in (False, True):
+        dec.use_mk = mk
+        print(f"decode from position {start}, one-launch step {mk}, w8a8={w8a8}", flush=True)
+        dec.prefill(img, prompt)
+        dec.start_decode()
+        lg = []
+        for _ in range(6):
+            dec.decode_step(logits=True)
+            lg.append(dec.logits.float().cpu().clone())
+        out[mk] = (dec.tokens[:7].cpu().tolist(), lg, dec.xd[0].cpu().clone())
+    assert dec.mk_error() == 0 and dec.mk_fallbacks == 0 and dec.state.cpu().tolist() == [7, start + 6]
+    compare_free_running(out, 2e-2 if w8a8 else 5e-3)
+
+
 YES, NO = [11, 222, 3333, 44444], [55, 666, 7777, 50000]
 
 
