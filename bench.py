@@ -33,11 +33,11 @@ def vision_flops_per_frame(layers=27, T=729, D=1152, F=4304, H=16, hd=72, Kp=588
 
 # LDS ring depth of each GEMM tile config (the kernel template's last argument)
 GEMM_STAGES = {0: 4, 1: 4, 2: 4, 3: 4, 4: 3, 5: 3, 6: 3, 7: 2, 8: 4, 9: 4, 10: 4, 11: 3, 12: 2, 13: 6, 14: 2,
-               15: 2, 16: 3, 17: 3, 18: 2, 19: 4, 20: 4, 21: 4, 22: 4, 23: 4, 24: 3, 25: 2, 26: 4, 27: 4}
+               16: 3, 18: 2, 20: 4, 21: 4, 22: 4, 23: 4, 24: 3, 26: 4}
 # wave grid (WGM, WGN) of the kind-0 configs that do not use 2 x 2
-GEMM_WAVES = {16: (4, 2), 17: (2, 4), 23: (1, 4)}
+GEMM_WAVES = {16: (4, 2), 23: (1, 4)}
 # 2 x 2 tiles over two k groups of waves (8 waves)
-GEMM_KH2 = {19, 20, 21, 22, 24, 26, 27}
+GEMM_KH2 = {20, 21, 22, 24, 26}
 
 
 def gemm_symbol(cfg):
@@ -50,6 +50,8 @@ def gemm_symbol(cfg):
         return f"gemm_bf16_kh2_kernel<{bm}, {bn}, {GEMM_STAGES[cfg]}>"
     if cfg in (15, 25):
         return f"gemm_big_kernel<{bn}>"
+    if cfg in (17, 19, 27):
+        return f"gemm_mid_kernel<{bn}>"
     wgm, wgn = GEMM_WAVES.get(cfg, (2, 2))
     return f"gemm_bf16_kernel<{bm}, {bn}, {wgm}, {wgn}, {GEMM_STAGES[cfg]}>"
 

@@ -34,6 +34,7 @@
 #include "common.h"
 #include "gemm_big.h"
 #include "gemm_epi.h"
+#include "gemm_mid.h"
 
 namespace {
 
@@ -967,12 +968,12 @@ constexpr Cfg kCfgs[] = {{128, 128, 4, 1, 0, 4}, {64, 128, 4, 1, 0, 4}, {128, 64
                          {64, 64, 4, 2, 1, 4},   {64, 128, 4, 1, 1, 4},  {128, 64, 4, 1, 1, 4}, {64, 64, 3, 3, 1, 4},
                          {64, 96, 2, 3, 1, 4},   {64, 64, 6, 1, 1, 4},   {96, 64, 2, 3, 1, 4},
                          // 8-wave tiles for large grids: 2 waves per SIMD hide each other's LDS reads and barriers
-                         // (256 x 256 is gemm_big.hip's persistent tile in bf16, an 8-wave tile in int8)
+                         // (in bf16 256 x 256 is gemm_big.hip's persistent tile, 128 x 256 gemm_mid.hip's)
                          {256, 256, 2, 1, 0, 8}, {256, 128, 3, 1, 0, 8}, {128, 256, 3, 1, 0, 8},
                          // 4 waves of 128 x 128: 8 LDS reads per 16 MFMAs (LDS traffic at 3/4 of the MFMA time)
                          {256, 256, 2, 1, 0, 4},
                          // 8-wave forms of the 2 x 2 tiles, two k groups (kh = 2): batch-1 grids, one workgroup per
-                         // CU, whose k loop waits on LDS reads at the 4-wave rate
+                         // CU, whose k loop waits on LDS reads at the 4-wave rate (128 x 128: gemm_mid.hip in bf16)
                          {128, 128, 4, 1, 0, 8, 2}, {64, 128, 4, 1, 0, 8, 2}, {128, 64, 4, 1, 0, 8, 2},
                          {64, 64, 4, 2, 0, 8, 2},
                          // one wave row x 4 wave columns, 3 x 1 MFMA blocks per wave: 96-row tiles for M = 729
@@ -982,7 +983,7 @@ constexpr Cfg kCfgs[] = {{128, 128, 4, 1, 0, 4}, {64, 128, 4, 1, 0, 4}, {128, 64
                          // 3-stage ring (two stages in flight), and gemm_big.hip's persistent 256 x 192 tile
                          {192, 192, 3, 1, 0, 8, 2}, {256, 192, 2, 1, 0, 8},
                          // 730-row prompt-prefix GEMMs: 4 row tiles of 192 x 64 column tiles of 128 = 256 workgroups
-                         // for N = 8192; two k groups of 2 x 2 waves, 4-stage ring
+                         // for N = 8192; two k groups of 2 x 2 waves, 4-stage ring. 128 x 192: gemm_mid.hip
                          {192, 128, 4, 1, 0, 8, 2}, {128, 192, 4, 1, 0, 8, 2}};
 constexpr int kNCfg = sizeof(kCfgs) / sizeof(kCfgs[0]);
 
@@ -1235,16 +1236,20 @@ extern "C" int mx_gemm_bf16(hipStream_t st, int cfg, int splits, const uint16_t*
       break;
     }
     case 16: e = launch<256, 128, 4, 2, 3>(st, splits, A, lda, W, ldw, bias, R, ldr, r_rows, C, ldc, M, N, K, Kw, act, act_ncols, ws, cnt); break;
-    case 17: e = launch<128, 256, 2, 4, 3>(st, splits, A, lda, W, ldw, bias, R, ldr, r_rows, C, ldc, M, N, K, Kw, act, act_ncols, ws, cnt); break;
+    case 17: case 19: case 27: {
+      // the one-tile-per-CU tiles; what they do not take (rows of C or R not in whole 16-byte chunks) runs on the
+      // 128 x 128 tile of config 7: the same bits
+      const BigGemm g{A, lda, W, ldw, bias, R, ldr, r_rows, C, ldc, M, N, K, Kw, act_ncols};
+      e = gemm_mid_fits(act, g) ? launch_gemm_mid(st, kCfgs[cfg].bn, act, g) : L_(128, 128, 2);
+      break;
+    }
     case 18: e = L_(256, 256, 2); break;
 #define H_(BM, BN, S) launch_kh2<BM, BN, S>(st, splits, A, lda, W, ldw, bias, R, ldr, r_rows, C, ldc, M, N, K, Kw, act, act_ncols)
-    case 19: e = H_(128, 128, 4); break;
     case 20: e = H_(64, 128, 4); break;
     case 21: e = H_(128, 64, 4); break;
     case 22: e = H_(64, 64, 4); break;
     case 24: e = H_(192, 192, 3); break;
     case 26: e = H_(192, 128, 4); break;
-    case 27: e = H_(128, 192, 4); break;
 #define W_(BM, BN, S, OCC) launch_ks<BM, BN, S, OCC>(st, A, lda, W, ldw, bias, R, ldr, r_rows, C, ldc, M, N, K, Kw, act, act_ncols)
     case 8: e = W_(64, 64, 4, 2); break;
     case 9: e = W_(64, 128, 4, 1); break;
@@ -1443,17 +1448,22 @@ extern "C" int mx_gemm_bf16_partial(hipStream_t st, int cfg, int splits, const u
     case 2: e = L_(128, 64, 4); break;
     case 3: e = L_(64, 64, 4); break;
     case 4: e = L_(256, 128, 3); break;
-    case 5: e = L_(128, 256, 3); break;
     case 6: e = L_(64, 64, 3); break;
     case 7: e = L_(128, 128, 2); break;
     case 23: e = launch<96, 128, 1, 4, 4>(st, splits, A, lda, W, ldw, nullptr, nullptr, 0, 0, nullptr, 0, M, N, K, Kw, 0, 0, nullptr, nullptr, P, ldp, p_split); break;
 #define H_(BM, BN, S) launch_kh2<BM, BN, S>(st, splits, A, lda, W, ldw, nullptr, nullptr, 0, 0, nullptr, 0, M, N, K, Kw, 0, 0, P, ldp, p_split)
-    case 19: e = H_(128, 128, 4); break;
+    case 5: case 19: case 27: {
+      const BigGemm g{A, lda, W, ldw, nullptr, nullptr, 0, 0, nullptr, 0, M, N, K, Kw, 0};
+      if (lda >= 1L << 21 || ldw >= 1L << 21)
+        e = L_(128, 128, 2);
+      else
+        e = launch_gemm_mid(st, kCfgs[cfg].bn, 0, g, splits, P, ldp, p_split);
+      break;
+    }
     case 20: e = H_(64, 128, 4); break;
     case 21: e = H_(128, 64, 4); break;
     case 22: e = H_(64, 64, 4); break;
     case 26: e = H_(192, 128, 4); break;
-    case 27: e = H_(128, 192, 4); break;
 #undef H_
     case 8: e = W_(64, 64, 4, 2); break;
     case 9: e = W_(64, 128, 4, 1); break;

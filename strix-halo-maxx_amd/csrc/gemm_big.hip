@@ -27,41 +27,13 @@
 //   20480 x 6144 x 768, gated GELU  217 ->  192
 //   9477 x 3456 x 1152             84.9 -> 71.6
 //   8192 x 8192 x 8192              851 ->  770 (1427 TFLOP/s)
-#include "gemm_big.h"
-
-#include "gemm_epi.h"
+#include "gemm_out.h"
 
 namespace {
-
-// 64 lanes x 16 bytes through a buffer resource (per-lane byte offset + wave-uniform offset; lanes outside the resource
-// read zeros) into LDS at lds + LO + 16 * lane.
-template <int LO>
-__device__ __forceinline__ void dma16b(u32x4 rsrc, uint32_t voff, uint32_t soff, uint32_t lds) {
-  asm volatile("s_add_u32 m0, %3, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(rsrc),
-               "s"(soff), "s"(lds), "n"(LO)
-               : "memory", "m0", "scc");
-}
 
 constexpr int BM = 256;
 constexpr int BK = 64;   // k columns per step
 constexpr int NW = 4;    // waves, 2 x 2
-
-// f(IntC<0>), .., f(IntC<N - 1>)
-template <int N, int n = 0, typename F>
-__device__ __forceinline__ void for_each(F&& f) {
-  if constexpr (n < N) {
-    f(IntC<n>{});
-    for_each<N, n + 1>(f);
-  }
-}
-
-// Piece n of a wave's write-out (32 rows x 64 columns, the last of a row of pieces 32 columns if FN is odd): its
-// 32-column blocks, its 16-byte chunks per output row, the rows of one store instruction
-template <int FN, bool GLU, int n>
-struct Piece {
-  static constexpr int blocks = FN - n % ((FN + 1) / 2) * 2 < 2 ? 1 : 2;
-  static constexpr int cpr = (GLU ? 2 : 4) * blocks, rpi = 64 / cpr;
-};
 
 template <int BN, int ACT, int HR, bool LIM>
 __global__ __launch_bounds__(256, 1) void gemm_big_kernel(BigGemm p, int tiles_m, int tiles_n) {
@@ -70,7 +42,6 @@ __global__ __launch_bounds__(256, 1) void gemm_big_kernel(BigGemm p, int tiles_m
   static_assert(FM == 4 && (FN == 3 || FN == 4), "four phases per step");
   constexpr bool GLU = ACT == 3;
   constexpr int LPS = 2 * (FM + FN);                          // load instructions per wave and step
-  constexpr int NPC = (FN + 1) / 2;                           // write-out pieces (32 rows x 64 columns) per 32 rows
   constexpr int NST = FM * FN * (GLU ? 1 : 2);                 // store instructions per wave and tile
   // LDS: two A slots, two W slots at 32 KB steps, the bias rows of up to 4 tiles, 4 KB of staging per wave
   constexpr int SLOT = 32 * 1024, W_O = 2 * SLOT, W_B = BN * BK * 2;
@@ -306,7 +277,6 @@ __global__ __launch_bounds__(256, 1) void gemm_big_kernel(BigGemm p, int tiles_m
   for (int s = 0; s < 4; s++) read_a(0, 0, s);
   flip(wa);
 
-  const int Ncols = GLU ? p.N / 2 : p.N;
   uint8_t* st = smem + EPI_O + wave * 4096;
   int bias_row = 0;
   for (int t = t0; t < run1; t += stride) {
@@ -319,106 +289,7 @@ __global__ __launch_bounds__(256, 1) void gemm_big_kernel(BigGemm p, int tiles_m
     const float* brow = reinterpret_cast<const float*>(smem + BIAS_O + bias_row * 1024);
     bias_row = (bias_row + 1) & 3;
 
-    // ---- write-out, per wave and without barriers: pieces of 32 rows x 64 columns (the last one 32 columns wide if
-    // FN is odd) through the wave's own 4 KB. Rows of 128 bytes, 16-byte chunks swizzled by ((row >> 1) & 7), their
-    // 8-byte halves swapped in rows 16 .. 31. A piece is computed while the one before it settles in the LDS and the one
-    // before that is sent.
-    int ln = lane;
-    asm volatile("" : "+v"(ln));  // the lane's addresses are computed here, per tile: hoisted they would spill
-    const int lr = ln & 31, hk = ln >> 5;
-    const uint32_t put_o = lr * 128 + (((lr >> 1) & 7) << 4) + ((GLU ? (lr >> 4) & 1 : hk ^ ((lr >> 4) & 1)) << 3) + (GLU ? 4 * hk : 0);
-    const int nw = cn0 + wn * WTN, oc = GLU ? nw / 2 : nw;  // first column of W / of the output
-    const long obytes = ((long)(p.M - cm0 - 1) * p.ldc + Ncols - (GLU ? cn0 / 2 : cn0)) * 2;
-    const uint64_t cu = (uint64_t)(uintptr_t)(p.C + (long)cm0 * p.ldc + (GLU ? cn0 / 2 : cn0));
-    uint16_t* cp = reinterpret_cast<uint16_t*>(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(cu >> 32)) << 32) |
-                                               (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)cu));
-    const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(
-        cp, (short)0, __builtin_amdgcn_readfirstlane((int)(obytes < 0x7ffffff0L ? obytes : 0x7ffffff0L)), 0x00020000);
-    constexpr int NP = FM * NPC;
-    u32x4 rr[HR ? NP : 1][4];
-    if constexpr (HR == 1) {
-      for_each<NP>([&](auto nc) {
-        constexpr int n = decltype(nc)::value, cpr = Piece<FN, GLU, n>::cpr, rpi = Piece<FN, GLU, n>::rpi;
-#pragma unroll
-        for (int u = 0; u < 32 / rpi; u++) {
-          int rm = min(cm0 + wm * WTM + n / NPC * 32 + u * rpi + ln / cpr, p.M - 1);
-          if (p.r_rows > 0) rm %= p.r_rows;
-          rr[n][u] = *reinterpret_cast<const u32x4*>(p.R + (long)rm * p.ldr + min(nw + n % NPC * 64 + ln % cpr * 8, p.N - 8));
-        }
-      });
-    }
-    f32x4 bv[FN][4];
-#pragma unroll
-    for (int i = 0; i < FN; i++)
-#pragma unroll
-      for (int g = 0; g < 4; g++) bv[i][g] = *reinterpret_cast<const f32x4*>(brow + wn * WTN + i * 32 + 8 * g + 4 * hk);
-    u32x2 ov[2][8];
-    u32x4 gv[2][4];
-    auto compute = [&](auto nc) {
-      constexpr int n = decltype(nc)::value;
-#pragma unroll
-      for (int ii = 0; ii < Piece<FN, GLU, n>::blocks; ii++)
-#pragma unroll
-        for (int g = 0; g < 4; g++) {
-          const int i = n % NPC * 2 + ii;
-          const f32x16& a = acc[i][n / NPC];
-          const f32x4 a4 = {a[4 * g], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]}, &b = bv[i][g];
-          if constexpr (ACT == 0)
-            ov[n & 1][4 * ii + g] = u32x2{pack2(a4[0] + b[0], a4[1] + b[1]), pack2(a4[2] + b[2], a4[3] + b[3])};
-          else
-            ov[n & 1][4 * ii + g] = epi_val<ACT, false, 0>(a4, b, u32x2{0u, 0u}, false, nw + i * 32 + 8 * g + 4 * hk,
-                                                           LIM ? p.act_ncols : 0);
-        }
-    };
-    auto put = [&](auto nc) {
-      constexpr int n = decltype(nc)::value;
-#pragma unroll
-      for (int ii = 0; ii < Piece<FN, GLU, n>::blocks; ii++)
-#pragma unroll
-        for (int g = 0; g < 4; g++)
-          if constexpr (GLU)
-            *reinterpret_cast<uint32_t*>(st + (put_o ^ ((2 * ii + (g >> 1)) << 4) ^ ((g & 1) << 3))) = ov[n & 1][4 * ii + g].x;
-          else
-            *reinterpret_cast<u32x2*>(st + (put_o ^ ((4 * ii + g) << 4))) = ov[n & 1][4 * ii + g];
-    };
-    auto get = [&](auto nc) {
-      constexpr int n = decltype(nc)::value, cpr = Piece<FN, GLU, n>::cpr, rpi = Piece<FN, GLU, n>::rpi;
-#pragma unroll
-      for (int u = 0; u < 32 / rpi; u++) {
-        const int r = u * rpi + ln / cpr;
-        gv[n & 1][u] = *reinterpret_cast<const u32x4*>(st + r * 128 + (((ln % cpr) ^ ((r >> 1) & 7)) << 4));
-      }
-    };
-    auto send = [&](auto nc) {
-      constexpr int n = decltype(nc)::value, cpr = Piece<FN, GLU, n>::cpr, rpi = Piece<FN, GLU, n>::rpi;
-      constexpr int c = n % NPC * (GLU ? 32 : 64);  // the piece's first output column in the wave's part
-      uint32_t vo = (uint32_t)(ln / cpr * p.ldc * 2 + ln % cpr * 16);
-      vo = oc + c + ln % cpr * 8 < Ncols ? vo : 0x80000000u;
-#pragma unroll
-      for (int u = 0; u < 32 / rpi; u++) {
-        u32x4 v = gv[n & 1][u];
-        if (rpi == 32 ? (ln / cpr) >> 4 & 1 : u * rpi >= 16) v = u32x4{v.z, v.w, v.x, v.y};
-        if constexpr (HR == 1) {
-#pragma unroll
-          for (int e = 0; e < 4; e++)
-            v[e] = pack2(lo_bf(v[e]) + lo_bf(rr[n][u][e]), hi_bf(v[e]) + hi_bf(rr[n][u][e]));
-        }
-        __builtin_amdgcn_raw_buffer_store_b128(
-            v, rc, vo, (wm * WTM + n / NPC * 32 + u * rpi) * (int)p.ldc * 2 + ((GLU ? wn * WTN / 2 : wn * WTN) + c) * 2, 0);
-      }
-    };
-    for_each<NP + 2>([&](auto nc) {
-      constexpr int n = decltype(nc)::value;
-      if constexpr (n < NP) compute(nc);
-      __builtin_amdgcn_sched_barrier(0);
-      if constexpr (n >= 2) send(IntC<n - 2>{});
-      __builtin_amdgcn_sched_barrier(0);
-      if constexpr (n >= 1 && n <= NP) get(IntC<n - 1>{});
-      asm volatile("" ::: "memory");  // a wave's LDS accesses complete in order: the reads see its own writes
-      if constexpr (n < NP) put(nc);
-      asm volatile("" ::: "memory");
-      __builtin_amdgcn_sched_barrier(0);
-    });
+    write_out<FM, FN, ACT, HR, LIM>(p, acc, cm0, cn0, wm * WTM, wn * WTN, brow, st, lane);
     after = 3;
     cm0 = nm0;
     cn0 = nn0;
