@@ -18,12 +18,14 @@ F = ctypes.c_float
 # name -> argtypes (every entry point returns int status)
 SIGNATURES = {
     "mx_gemm_bf16": [P, I, I, P, L, P, L, P, P, L, I, P, L, I, I, I, I, I, I, P, L, P, L],
+    "mx_gemm_bf16_act_from": [P, I, I, P, L, P, L, P, P, L, I, P, L, I, I, I, I, I, I, P, L, P, L],
     "mx_gemm_check": [I, I, P, L, P, L, P, P, L, P, L, I, I, I, I, I, P, L, P, L],
     "mx_gemm_pick": [I, I, I],
     "mx_gemm_ws_elems": [I, I, I, I],
     "mx_track_head_blob_elems": [I, I, I],
     "mx_resize_patchify_u8": [P, P, I, I, P, L, I, I, I],
     "mx_gemm_reduce": [P, P, I, L, L, P, P, L, I, P, L, I, I, I, I],
+    "mx_gemm_reduce_act_from": [P, P, I, L, L, P, P, L, I, P, L, I, I, I, I],
     "mx_gemm_i8_partial": [P, I, I, P, L, P, L, P, L, L, I, I, I, I],
     "mx_gemm_i8_reduce": [P, P, I, L, L, P, P, P, P, L, I, P, L, I, I, I],
     "mx_ssm_step_rows": [P, P, P, P, P, L, P, L, P, P, P, P, P, P, P, P, P, P, L, I, I, P, P, I, P, L],

@@ -1195,16 +1195,11 @@ extern "C" int mx_gemm_check(int cfg, int splits, const void* A, long lda, const
   return MX_OK;
 }
 
-// C = epi(A W^T + bias). cfg < 0: the library's pick (only split-free picks unless a workspace is given).
-// ws / cnt: split-K workspace (fp32 elements) and per-tile counters (must be zero before first use; the kernel
-// leaves them zero). R row for output row m is (r_rows > 0 ? m % r_rows : m).
-// act: 0 none, 1 GELU-tanh, 2 GELU-erf, 3 gated GELU-tanh on interleaved (gate, up) weight-row pairs (output width
-// N / 2: column j = bf16(bf16(gelu(gate_j)) * up_j) with gate_j / up_j = linear rows 2 j / 2 j + 1). act 1-2 apply
-// to output columns < act_ncols only when act_ncols > 0 (e.g. GELU on the y half of a fused [y | x] projection).
-extern "C" int mx_gemm_bf16(hipStream_t st, int cfg, int splits, const uint16_t* A, long lda, const uint16_t* W,
-                            long ldw, const float* bias, const uint16_t* R, long ldr, int r_rows, uint16_t* C,
-                            long ldc, int M, int N, int K, int Kw, int act, int act_ncols, float* ws, long ws_elems,
-                            int* cnt, long n_cnt) {
+namespace {
+// mx_gemm_bf16 with act_ncols as epi_val reads it (negative: the activation applies from column -act_ncols on).
+int gemm_bf16(hipStream_t st, int cfg, int splits, const uint16_t* A, long lda, const uint16_t* W, long ldw,
+              const float* bias, const uint16_t* R, long ldr, int r_rows, uint16_t* C, long ldc, int M, int N, int K,
+              int Kw, int act, int act_ncols, float* ws, long ws_elems, int* cnt, long n_cnt) {
   if (r_rows < 0) return MX_ESHAPE;
   if (cfg < 0) {
     const int p = mx_gemm_pick(M, N, Kw);
@@ -1264,6 +1259,32 @@ extern "C" int mx_gemm_bf16(hipStream_t st, int cfg, int splits, const uint16_t*
 #undef W_
 #undef H_
   return e == hipSuccess ? MX_OK : MX_ELAUNCH;
+}
+}  // namespace
+
+// C = epi(A W^T + bias). cfg < 0: the library's pick (only split-free picks unless a workspace is given).
+// ws / cnt: split-K workspace (fp32 elements) and per-tile counters (must be zero before first use; the kernel
+// leaves them zero). R row for output row m is (r_rows > 0 ? m % r_rows : m).
+// act: 0 none, 1 GELU-tanh, 2 GELU-erf, 3 gated GELU-tanh on interleaved (gate, up) weight-row pairs (output width
+// N / 2: column j = bf16(bf16(gelu(gate_j)) * up_j) with gate_j / up_j = linear rows 2 j / 2 j + 1). act 1-2 apply
+// to output columns < act_ncols only when act_ncols > 0 (e.g. GELU on the y half of a fused [y | x] projection).
+extern "C" int mx_gemm_bf16(hipStream_t st, int cfg, int splits, const uint16_t* A, long lda, const uint16_t* W,
+                            long ldw, const float* bias, const uint16_t* R, long ldr, int r_rows, uint16_t* C,
+                            long ldc, int M, int N, int K, int Kw, int act, int act_ncols, float* ws, long ws_elems,
+                            int* cnt, long n_cnt) {
+  return gemm_bf16(st, cfg, splits, A, lda, W, ldw, bias, R, ldr, r_rows, C, ldc, M, N, K, Kw, act,
+                   act_ncols > 0 ? act_ncols : 0, ws, ws_elems, cnt, n_cnt);
+}
+
+// The same with the activation on columns >= act_from only (act 1, 2): the GELU of fc1's columns in one product over the
+// fused [qkv | fc1] rows.
+extern "C" int mx_gemm_bf16_act_from(hipStream_t st, int cfg, int splits, const uint16_t* A, long lda,
+                                     const uint16_t* W, long ldw, const float* bias, const uint16_t* R, long ldr,
+                                     int r_rows, uint16_t* C, long ldc, int M, int N, int K, int Kw, int act,
+                                     int act_from, float* ws, long ws_elems, int* cnt, long n_cnt) {
+  if (act_from < 0 || act == 3) return MX_EBADCFG;
+  return gemm_bf16(st, cfg, splits, A, lda, W, ldw, bias, R, ldr, r_rows, C, ldc, M, N, K, Kw, act, -act_from, ws,
+                   ws_elems, cnt, n_cnt);
 }
 
 // ---------------------------------------------------------------------------------------------- allocation-free form
@@ -1334,15 +1355,9 @@ extern "C" int mx_gemm_bf16_noalloc(hipStream_t st, int cfg, int splits, const u
                       splits > 1 ? kScratchWs : 0, cnt, splits > 1 ? kScratchCnt : 0);
 }
 
-// C = epi(sum over s < nsplit of P[s] + bias): the epilogue of mx_gemm_bf16 (act 0 / 1 / 2 on columns < act_ncols when
-// act_ncols > 0, 3 = gated GELU on interleaved (gate, up) column pairs with output width N / 2; then + R) on raw
-// partials from mx_gemm_bf16_partial, splits added in order. Partial GEMM + this reduction is the fence-free
-// split-K: no counters, no cross-workgroup visibility inside a launch (stream order is the only synchronisation).
-// No counterpart in the reference; it stands for the small-M split-K path of i8gemm_small_launch
-// (moondream/gpu/hip/i8gemm.hip:555-592) on the bf16 side.
-extern "C" int mx_gemm_reduce(hipStream_t st, const float* P, int nsplit, long p_split, long ldp, const float* bias,
-                              const uint16_t* R, long ldr, int r_rows, uint16_t* C, long ldc, int M, int N, int act,
-                              int act_ncols) {
+namespace {
+int gemm_reduce(hipStream_t st, const float* P, int nsplit, long p_split, long ldp, const float* bias,
+                const uint16_t* R, long ldr, int r_rows, uint16_t* C, long ldc, int M, int N, int act, int act_ncols) {
   if (!P || !C) return MX_ENULL;
   if (nsplit < 1 || nsplit > 64 || M < 1 || N < 4 || N % 4 || ldp % 4 || ldp < N || act < 0 || act > 3 ||
       r_rows < 0 || (nsplit > 1 && p_split < (long)M * ldp) || p_split % 4)
@@ -1361,6 +1376,27 @@ extern "C" int mx_gemm_reduce(hipStream_t st, const float* P, int nsplit, long p
   }
 #undef RL_
   return hipGetLastError() == hipSuccess ? MX_OK : MX_ELAUNCH;
+}
+}  // namespace
+
+// C = epi(sum over s < nsplit of P[s] + bias): the epilogue of mx_gemm_bf16 (act 0 / 1 / 2 on columns < act_ncols when
+// act_ncols > 0, 3 = gated GELU on interleaved (gate, up) column pairs with output width N / 2; then + R) on raw
+// partials from mx_gemm_bf16_partial, splits added in order. Partial GEMM + this reduction is the fence-free
+// split-K: no counters, no cross-workgroup visibility inside a launch (stream order is the only synchronisation).
+// No counterpart in the reference; it stands for the small-M split-K path of i8gemm_small_launch
+// (moondream/gpu/hip/i8gemm.hip:555-592) on the bf16 side.
+extern "C" int mx_gemm_reduce(hipStream_t st, const float* P, int nsplit, long p_split, long ldp, const float* bias,
+                              const uint16_t* R, long ldr, int r_rows, uint16_t* C, long ldc, int M, int N, int act,
+                              int act_ncols) {
+  return gemm_reduce(st, P, nsplit, p_split, ldp, bias, R, ldr, r_rows, C, ldc, M, N, act, act_ncols > 0 ? act_ncols : 0);
+}
+
+// The same with the activation on columns >= act_from only (mx_gemm_bf16_act_from's epilogue).
+extern "C" int mx_gemm_reduce_act_from(hipStream_t st, const float* P, int nsplit, long p_split, long ldp,
+                                       const float* bias, const uint16_t* R, long ldr, int r_rows, uint16_t* C,
+                                       long ldc, int M, int N, int act, int act_from) {
+  if (act_from < 0 || act == 3) return MX_EBADCFG;
+  return gemm_reduce(st, P, nsplit, p_split, ldp, bias, R, ldr, r_rows, C, ldc, M, N, act, -act_from);
 }
 
 // W8A8 split-K: raw int32 partials of S splits of the int8 GEMM (the same tile kernel in its raw mode, each split a

@@ -311,7 +311,7 @@ hipError_t launch_bn(hipStream_t st, int act, const BigGemm& g) {
     hipLaunchKernelGGL(kern, grid, blk, 0, st, g, tm, tn);
     return hipGetLastError();
   };
-  const bool lim = g.act_ncols > 0 && g.act_ncols < g.N;
+  const bool lim = g.act_ncols != 0 && g.act_ncols < g.N;
   if (g.R) {
     if (act == 0) return go(gemm_big_kernel<BN, 0, 1, false>);
     if (act == 1) return lim ? go(gemm_big_kernel<BN, 1, 1, true>) : go(gemm_big_kernel<BN, 1, 1, false>);

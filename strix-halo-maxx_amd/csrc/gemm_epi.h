@@ -23,7 +23,7 @@ __device__ __forceinline__ void tile_of(int b, int tiles_m, int tiles_n, int spl
 }
 
 // Epilogue of one 4-column group (output row m, columns n .. n+3) from fp32 sums s: + bias, round to bf16, activation
-// ACT (1 GELU-tanh, 2 GELU-erf; rounded again; skipped for columns >= act_ncols when act_ncols > 0), + residual
+// ACT (1 GELU-tanh, 2 GELU-erf; rounded again; act_ncols > 0: on columns < act_ncols, < 0: >= -act_ncols), + residual
 // (fp32 add, rounded once more). ACT 3 is the gated GELU of interleaved (gate, up) column pairs, written to columns
 // n / 2, n / 2 + 1.
 template <int V>
@@ -48,7 +48,7 @@ __device__ __forceinline__ u32x2 epi_val(const f32x4& s, const f32x4& bv, const 
       v[e] = t * sw[e] + bv[e];
     }
     if constexpr (ACT == 1 || ACT == 2) {
-      const bool on = act_ncols <= 0 || n < act_ncols;
+      const bool on = act_ncols <= 0 ? n >= -act_ncols : n < act_ncols;
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         const float g = ACT == 1 ? gelu_tanh(v[e]) : gelu_erf(v[e]);
@@ -72,7 +72,7 @@ __device__ __forceinline__ u32x2 epi_val(const f32x4& s, const f32x4& bv, const 
   } else {
     if constexpr (ACT == 1 || ACT == 2) {
       // the activation's bf16 rounding: explicit before a residual add, else the final pack's own rounding
-      const bool on = act_ncols <= 0 || n < act_ncols;
+      const bool on = act_ncols <= 0 ? n >= -act_ncols : n < act_ncols;
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         float g = ACT == 1 ? gelu_tanh(v[e]) : gelu_erf(v[e]);

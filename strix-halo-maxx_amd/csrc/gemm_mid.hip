@@ -169,7 +169,7 @@ hipError_t launch_bn(hipStream_t st, int act, const BigGemm& g, int splits, floa
     return hipGetLastError();
   };
   if (P) return go(gemm_mid_kernel<BN, 0, 0, false, true>);
-  const bool lim = g.act_ncols > 0 && g.act_ncols < g.N;
+  const bool lim = g.act_ncols != 0 && g.act_ncols < g.N;
   if (g.R) {
     if (act == 0) return go(gemm_mid_kernel<BN, 0, 1, false, false>);
     if (act == 1) return lim ? go(gemm_mid_kernel<BN, 1, 1, true, false>) : go(gemm_mid_kernel<BN, 1, 1, false, false>);

@@ -123,7 +123,7 @@ class MxLin:
         self.cfgs = {}  # M -> (cfg, splits); absent: tuned (or library pick) on first use
         self.dev = self.w.device
 
-    def _launch(self, cfg, splits, x2, y2, M, a, r2, ldr, r_rows, ws, act_cols=0):
+    def _launch(self, cfg, splits, x2, y2, M, a, r2, ldr, r_rows, ws, act_cols=0, act_from=0):
         """splits > 0: mx_gemm_bf16 (in-kernel split-K when > 1); splits = -S: the fence-free split-K, raw partials of
         S splits into the workspace (mx_gemm_bf16_partial) then the epilogue over their sum (mx_gemm_reduce)."""
         lib = _lib.load()
@@ -135,11 +135,13 @@ class MxLin:
             rc = _partial(self, cfg, S, x2, P, M)
             if rc != 0:
                 return rc
-            return lib.mx_gemm_reduce(stream(), P.data_ptr(), S, M * N, N, ptr(self.b), ptr(r2), ldr, r_rows,
-                                      y2.data_ptr(), y2.stride(0), M, N, a, act_cols)
-        return lib.mx_gemm_bf16(
+            fn = lib.mx_gemm_reduce_act_from if act_from else lib.mx_gemm_reduce
+            return fn(stream(), P.data_ptr(), S, M * N, N, ptr(self.b), ptr(r2), ldr, r_rows, y2.data_ptr(),
+                      y2.stride(0), M, N, a, act_from or act_cols)
+        fn = lib.mx_gemm_bf16_act_from if act_from else lib.mx_gemm_bf16
+        return fn(
             stream(), cfg, splits, x2.data_ptr(), x2.stride(0), self.w.data_ptr(), self.w.stride(0), ptr(self.b),
-            ptr(r2), ldr, r_rows, y2.data_ptr(), y2.stride(0), M, self.N, self.K, self.Kw, a, act_cols,
+            ptr(r2), ldr, r_rows, y2.data_ptr(), y2.stride(0), M, self.N, self.K, self.Kw, a, act_from or act_cols,
             ptr(ws.ws), ws.ws.numel(), ptr(ws.cnt), ws.cnt.numel())
 
     def _pick(self, M, x2, y2, a, r2, ldr, r_rows, ws):
@@ -158,9 +160,12 @@ class MxLin:
         _TUNED[key] = c
         return c
 
-    def __call__(self, x, gelu=False, res=None, pre=None, act=None, out=None, act_cols=0):
+    def __call__(self, x, gelu=False, res=None, pre=None, act=None, out=None, act_cols=0, act_from=0):
         """act: None / "tanh" / "erf" / "glu" (gated GELU on interleaved (gate, up) weight rows: output width N / 2);
-        act_cols > 0 limits the activation to output columns < act_cols."""
+        act_cols > 0 limits the activation to output columns < act_cols, act_from > 0 to columns >= act_from (not both,
+        and not with "glu")."""
+        if act_from and (act_cols > 0 or act == "glu"):
+            raise ValueError("act_from goes with neither act_cols nor glu")
         a = ACT[act if act is not None else gelu]
         Nout = self.N // 2 if a == 3 else self.N
         x2 = _rows(x, self.K)
@@ -191,7 +196,7 @@ class MxLin:
             ws.reserve(*_ws_need(cfg, splits, M, self.N))
         elif splits < 0:
             ws.reserve(-splits * M * self.N, 0)
-        _lib.check(self._launch(cfg, splits, x2, y2, M, a, r2, ldr, r_rows, ws, act_cols), "mx_gemm_bf16")
+        _lib.check(self._launch(cfg, splits, x2, y2, M, a, r2, ldr, r_rows, ws, act_cols, act_from), "mx_gemm_bf16")
         return y2.view(*x.shape[:-1], Nout) if out is None else y
 
     def partial(self, x, out=None):
