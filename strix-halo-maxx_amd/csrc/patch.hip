@@ -9,6 +9,57 @@
 
 namespace {
 
+// The normalised value of a byte (256 of them: every operation of the mode, once per value).
+__device__ __forceinline__ uint16_t norm_u8(float u, int mode) {
+  if (mode == 0) {
+    const float a = rbf(u / 255.0f);
+    return f2bf(rbf(a - 0.5f) * 2.0f);
+  }
+  return f2bf(__fsub_rn(__fdiv_rn(u, 127.5f), 1.0f));
+}
+
+// Thread -> 8 consecutive columns of one patch row (one 16-byte store): the column is split into (c, ky, kx) once and
+// stepped, and the normalisation is a look-up in LDS. One element per thread, with its own 64-bit divisions by ldo and
+// an IEEE division, spent its time on those (us, before -> now: 1 crop of 378 x 378 4.2 -> 3.5, 13 crops, 17 MB,
+// 27.4 -> 10.6, 256 crops 365 -> 125). Grid: x over an image's chunks (below 2^31), y over the images.
+__global__ __launch_bounds__(256) void patchify8_kernel(const uint8_t* __restrict__ img, uint16_t* __restrict__ out,
+                                                        int ldo, int B, int S, int P, int mode) {
+  __shared__ uint16_t tab[256];
+  tab[threadIdx.x] = norm_u8((float)threadIdx.x, mode);
+  __syncthreads();
+  const int G = S / P, K = 3 * P * P, nch = ldo >> 3;
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  if (i >= (uint32_t)(G * G) * nch) return;
+  const uint32_t p = i / (uint32_t)nch;
+  const int k0 = (int)(i - p * nch) * 8;
+  const int gy = (int)p / G, gx = (int)p - gy * G;
+  const int c0 = k0 / (P * P), r0 = k0 - c0 * (P * P), ky0 = r0 / P, kx0 = r0 - ky0 * P;
+  for (int b = blockIdx.y; b < B; b += gridDim.y) {
+    const uint8_t* src = img + (((long)b * S + gy * P) * S + gx * P) * 3;
+    int c = c0, ky = ky0, kx = kx0;
+    uint32_t u[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      const bool in = k0 + e < K;
+      u[e] = src[in ? ((long)ky * S + kx) * 3 + c : 0];
+      if (++kx == P) {
+        kx = 0;
+        if (++ky == P) {
+          ky = 0;
+          c++;
+        }
+      }
+    }
+    u32x4 o;
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+      o[e] = (k0 + 2 * e < K ? (uint32_t)tab[u[2 * e]] : 0u) | (k0 + 2 * e + 1 < K ? (uint32_t)tab[u[2 * e + 1]] << 16 : 0u);
+    *reinterpret_cast<u32x4*>(out + ((long)b * G * G + p) * ldo + k0) = o;
+  }
+}
+
+// The same one element per thread: rows that are not whole aligned 16-byte chunks, and grids of fewer than 32768 of
+// them, where the eight loads of a thread cost more than its divisions save (one 256 x 256 frame: 3.0 against 3.2 us).
 __global__ __launch_bounds__(256) void patchify_kernel(const uint8_t* __restrict__ img, uint16_t* __restrict__ out,
                                                        long ldo, int B, int S, int P, int mode) {
   const int G = S / P, K = 3 * P * P;
@@ -21,13 +72,7 @@ __global__ __launch_bounds__(256) void patchify_kernel(const uint8_t* __restrict
       const int b = (int)(row / (G * G)), p = (int)(row % (G * G));
       const int gy = p / G, gx = p % G;
       const int c = k / (P * P), r = k % (P * P), ky = r / P, kx = r % P;
-      const float u = (float)img[(((long)b * S + gy * P + ky) * S + gx * P + kx) * 3 + c];
-      if (mode == 0) {
-        const float a = rbf(u / 255.0f);
-        v = f2bf(rbf(a - 0.5f) * 2.0f);
-      } else {
-        v = f2bf(__fsub_rn(__fdiv_rn(u, 127.5f), 1.0f));
-      }
+      v = norm_u8((float)img[(((long)b * S + gy * P + ky) * S + gx * P + kx) * 3 + c], mode);
     }
     out[i] = v;
   }
@@ -99,6 +144,12 @@ extern "C" int mx_patchify_u8(hipStream_t st, const uint8_t* img, uint16_t* out,
                               int mode) {
   if (!img || !out) return MX_ENULL;
   if (B < 1 || P < 1 || S % P || ldo < 3L * P * P || mode < 0 || mode > 1) return MX_ESHAPE;
+  const long chunks = (long)(S / P) * (S / P) * (ldo / 8);
+  if (ldo % 8 == 0 && !((uintptr_t)out & 15) && ldo < (1L << 30) && chunks * B >= 32768 && chunks < 0x7fffffffL) {
+    hipLaunchKernelGGL(patchify8_kernel, dim3((unsigned)((chunks + 255) / 256), B < 65535 ? B : 65535), dim3(256), 0, st,
+                       img, out, (int)ldo, B, S, P, mode);
+    return hipGetLastError() == hipSuccess ? MX_OK : MX_ELAUNCH;
+  }
   const long total = (long)B * (S / P) * (S / P) * ldo;
   const int blocks = (int)((total + 255) / 256 < 65536 ? (total + 255) / 256 : 65536);
   hipLaunchKernelGGL(patchify_kernel, dim3(blocks), dim3(256), 0, st, img, out, ldo, B, S, P, mode);
