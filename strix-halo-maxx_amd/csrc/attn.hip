@@ -182,9 +182,6 @@ __global__ __launch_bounds__(64 * NQW * NKW) void attn_fwd_kernel(
     const uint8_t* Kst = smem + (kb % S) * C::STAGE_B + kw * KBW * ROWB;
     const uint8_t* Vst = smem + (kb % S) * C::STAGE_B + KB * ROWB + kw * KBW * ROWB;
 
-    // Head dim 64: a wave's MFMA phases go before the other waves' softmax phases (16 x 12 x 1280: 121 -> 116-118 us);
-    // head dim 72, where the exponentials of four waves per SIMD already fill the gaps: no difference (256 crops 1060).
-    if constexpr (D == 64) __builtin_amdgcn_s_setprio(1);
     // ---- S^T = K Q^T for NST x 32 keys (the NST chains interleave)
     f32x16 st[NST];
 #pragma unroll
@@ -201,7 +198,6 @@ __global__ __launch_bounds__(64 * NQW * NKW) void attn_fwd_kernel(
         const bf16x8 a = as_bf16x8(*reinterpret_cast<const u32x4*>(Kst + key * ROWB + slot * 16));
         st[kt] = mfma32(a, qf[s], st[kt]);
       }
-    if constexpr (D == 64) __builtin_amdgcn_s_setprio(0);
     // ---- mask, online softmax. Scores stay unscaled until the exponent: p = exp2(scale_log2 s - m) with m the
     // running max in scaled units. The running max is only raised (and O, l rescaled) when a query's block max
     // exceeds it by more than 8, i.e. the exponentials of a stale max stay <= 256; the normalisation at the end is
@@ -256,7 +252,6 @@ __global__ __launch_bounds__(64 * NQW * NKW) void attn_fwd_kernel(
     // ---- O^T += V^T P^T ; k-step (kt, s) covers keys kt*32 + 16 s + {4hk..4hk+3, 8+4hk..8+4hk+3}. The V^T
     // operand comes from two transpose reads: lane j = lane & 15 of each 16-lane group points at
     // V[first key + (j >> 2)][d0 + 4 (j & 3)], d0 = 32 dt + 16 ((lane >> 4) & 1).
-    if constexpr (D == 64) __builtin_amdgcn_s_setprio(1);
     const int jr = (lane & 15) >> 2, jc = 4 * (lane & 3) + 16 * ((lane >> 4) & 1);
 #pragma unroll
     for (int kt = 0; kt < NST; kt++)
@@ -287,7 +282,6 @@ __global__ __launch_bounds__(64 * NQW * NKW) void attn_fwd_kernel(
           oacc[dt] = mfma32(as_bf16x8(va), bp, oacc[dt]);
         }
       }
-    if constexpr (D == 64) __builtin_amdgcn_s_setprio(0);
   }
 
   if constexpr (NKW > 1) {
