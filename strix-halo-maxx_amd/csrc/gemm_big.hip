@@ -16,7 +16,7 @@
 //    through a private 4 KB of LDS per wave in three overlapped stages without barriers.
 // With one wave per SIMD every instruction between the MFMAs costs issue time (a 32 x 32 x 16 MFMA covers about 6
 // vector or 3 scalar instructions, measured), so the issue order is written out and the loads address memory through
-// buffer resources: no address arithmetic, and rows past the edge need no clamping. For the same reason the activation
+// buffer resources: one add per load, and rows past the edge need no clamping. For the same reason the activation
 // is not spread over the next tile's steps: 192 waiting values per lane and 10 instructions per value between the
 // MFMAs took longer than the write-out they would have hidden (qkv below: 1.35 ms).
 // Measured (us, before -> now; the 8-wave tile before, the better of both widths):
@@ -102,11 +102,11 @@ __global__ __launch_bounds__(256, 1) void gemm_big_kernel(BigGemm p, int tiles_m
     constexpr int j = decltype(jc)::value, e = decltype(ec)::value;
     if (j == 0 && e == 0 && ak == 0 && p.bias)  // the tile's bias row, by every wave to the same place
       dma16s(p.bias, (uint32_t)min(nn0 + 4 * lane, p.N - 4) * 4, sbase + BIAS_O + abias * 1024);
-    dma16b<(e * WTM + j * 32) * BK * 2>(ra, vak, (uint32_t)(4 * e + j) * a32, alds);
+    dma16b<(e * WTM + j * 32) * BK * 2>(ra, vak + (uint32_t)(4 * e + j) * a32, alds);
   };
   auto load_w = [&](auto ic, auto ec) {
     constexpr int i = decltype(ic)::value, e = decltype(ec)::value;
-    dma16b<(e * WTN + i * 32) * BK * 2>(rw, vwk, (uint32_t)(FN * e + i) * w32, wlds);
+    dma16b<(e * WTN + i * 32) * BK * 2>(rw, vwk + (uint32_t)(FN * e + i) * w32, wlds);
   };
   auto chunk_a = [&]() { vak = ak * BK + dch * 8 < p.K ? va + ak * (BK * 2) : 0x80000000u; };
   auto chunk_w = [&]() { vwk = vw + (wk * BK < p.Kw ? wk * (BK * 2) : 0x80000000u); };

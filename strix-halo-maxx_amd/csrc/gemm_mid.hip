@@ -74,9 +74,9 @@ __global__ __launch_bounds__(256, 1) void gemm_mid_kernel(BigGemm p, int tiles_m
   auto load = [&](auto ic, uint32_t so) {
     constexpr int i = decltype(ic)::value;
     if constexpr (i < LA)
-      dma16b<i * 4096>(ra, vak, (uint32_t)i * a32, lbase + so);
+      dma16b<i * 4096>(ra, vak + (uint32_t)i * a32, lbase + so);
     else
-      dma16b<i * 4096>(rw, vwk, (uint32_t)(i - LA) * w32, lbase + so);
+      dma16b<i * 4096>(rw, vwk + (uint32_t)(i - LA) * w32, lbase + so);
   };
 
   if (!PART && tid < 64) *reinterpret_cast<u32x4*>(smem + BIAS_O + tid * 16) = u32x4{0u, 0u, 0u, 0u};

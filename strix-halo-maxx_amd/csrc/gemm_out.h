@@ -6,12 +6,13 @@
 
 namespace {
 
-// 64 lanes x 16 bytes through a buffer resource (per-lane byte offset + wave-uniform offset; lanes outside the resource
-// read zeros) into LDS at lds + LO + 16 * lane.
+// 64 lanes x 16 bytes through a buffer resource (byte offset per lane; lanes outside the resource read zeros) into LDS at
+// lds + LO + 16 * lane. The whole offset is the lane's, rows included: the resource's range check covers it, while a
+// scalar offset beyond the resource's size (a row of the tile past a short matrix) is not what that check is for.
 template <int LO>
-__device__ __forceinline__ void dma16b(u32x4 rsrc, uint32_t voff, uint32_t soff, uint32_t lds) {
-  asm volatile("s_add_u32 m0, %3, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(rsrc),
-               "s"(soff), "s"(lds), "n"(LO)
+__device__ __forceinline__ void dma16b(u32x4 rsrc, uint32_t voff, uint32_t lds) {
+  asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(rsrc), "s"(lds),
+               "n"(LO)
                : "memory", "m0", "scc");
 }
 
@@ -112,7 +113,7 @@ __device__ __forceinline__ void write_out(const BigGemm& p, const f32x16 (&acc)[
   auto send = [&](auto nc) {
     constexpr int n = decltype(nc)::value, cpr = Piece<FN, GLU, n>::cpr, rpi = Piece<FN, GLU, n>::rpi;
     constexpr int c = n % NPC * (GLU ? 32 : 64);  // the piece's first output column in the wave's part
-    uint32_t vo = (uint32_t)(ln / cpr * p.ldc * 2 + ln % cpr * 16);
+    uint32_t vo = (uint32_t)((wr + n / NPC * 32 + ln / cpr) * p.ldc * 2 + ((GLU ? wc / 2 : wc) + c + ln % cpr * 8) * 2);
     vo = oc + c + ln % cpr * 8 < Ncols ? vo : 0x80000000u;
   #pragma unroll
     for (int u = 0; u < 32 / rpi; u++) {
@@ -123,8 +124,8 @@ __device__ __forceinline__ void write_out(const BigGemm& p, const f32x16 (&acc)[
         for (int e = 0; e < 4; e++)
           v[e] = pack2(lo_bf(v[e]) + lo_bf(rr[n][u][e]), hi_bf(v[e]) + hi_bf(rr[n][u][e]));
       }
-      __builtin_amdgcn_raw_buffer_store_b128(
-          v, rc, vo, (wr + n / NPC * 32 + u * rpi) * (int)p.ldc * 2 + ((GLU ? wc / 2 : wc) + c) * 2, 0);
+      // the row is in the lane's offset (as in dma16b): rows past M lie past the resource's end and are dropped
+      __builtin_amdgcn_raw_buffer_store_b128(v, rc, vo + (uint32_t)(u * rpi) * (uint32_t)p.ldc * 2u, 0, 0);
     }
   };
   for_each<NP + 2>([&](auto nc) {

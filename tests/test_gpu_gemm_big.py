@@ -1,5 +1,6 @@
 """The persistent 256-row GEMM (tile configs 15 and 25) against the 128 x 128 tile (config 7) on the same inputs: the same
-k order and roundings, so the same bits, for every epilogue and at the edges of its tiles and steps."""
+k order and roundings, so the same bits, for every epilogue and at the edges of its tiles and steps, with nothing written
+past a row's end or below the last row (256 guard rows: a whole tile)."""
 import pytest
 import torch
 
@@ -30,10 +31,11 @@ def test_big_tiles_equal_the_small_one(dev, cfg, M, N, K):
             got = []
             for c in (7, cfg):
                 lin.cfgs[M] = (c, 1)
-                y = torch.full((M, No + 8), 7.0, device=dev, dtype=BF)  # rows longer than the output: nothing past it changes
-                lin(x, out=y[:, :No], **kw)
+                y = torch.full((M + 256, No + 8), 7.0, device=dev, dtype=BF)  # longer and more rows than the output
+                lin(x, out=y[:M, :No], **kw)
                 got.append(y.cpu())
             assert torch.equal(got[0], got[1]), kw
+            assert torch.all(got[1][M:] == 7.0) and torch.all(got[1][:, No:] == 7.0), kw
 
 
 def test_big_tiles_take_what_the_config_took(dev):

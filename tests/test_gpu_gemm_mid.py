@@ -1,5 +1,6 @@
 """The one-tile-per-CU GEMM (tile configs 17, 19, 27, and 5 for partials) against the 128 x 128 tile (config 7) on the same
-inputs: the same k order and roundings, so the same bits, for every epilogue and at the edges of its tiles and steps."""
+inputs: the same k order and roundings, so the same bits, for every epilogue and at the edges of its tiles and steps, with
+nothing written past a row's end or below the last row (128 guard rows: a whole tile)."""
 import pytest
 import torch
 
@@ -30,16 +31,17 @@ def test_mid_tiles_equal_the_small_one(dev, cfg, M, N, K):
             got = []
             for c in (7, cfg):
                 lin.cfgs[M] = (c, 1)
-                y = torch.full((M, No + 8), 7.0, device=dev, dtype=BF)  # rows longer than the output: nothing past it changes
-                lin(x, out=y[:, :No], **kw)
+                y = torch.full((M + 128, No + 8), 7.0, device=dev, dtype=BF)  # longer and more rows than the output
+                lin(x, out=y[:M, :No], **kw)
                 got.append(y.cpu())
             assert torch.equal(got[0], got[1]), kw
+            assert torch.all(got[1][M:] == 7.0) and torch.all(got[1][:, No:] == 7.0), kw
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 12, 200), (129, 268, 904), (730, 2048, 1024)])
 @pytest.mark.parametrize("cfg", [5, 19, 27])
 def test_mid_partials_equal_the_small_ones(dev, cfg, M, N, K):
-    """Raw split-K partials in rows longer than N: the same bits as config 7's, nothing written past a row."""
+    """Raw split-K partials in rows longer than N: the same bits as config 7's, nothing written past or below the rows."""
     g = torch.Generator().manual_seed(M + N)
     x = torch.randn(M, K, generator=g).to(BF).to(dev)
     lin = ops.MxLin((torch.randn(N, K, generator=g) * 0.02).to(BF), None)
@@ -50,10 +52,11 @@ def test_mid_partials_equal_the_small_ones(dev, cfg, M, N, K):
         print(f"mid partial cfg={cfg} {M}x{N}x{K} splits={sp}", flush=True)
         out = []
         for c in (7, cfg):
-            P = torch.full((sp, M, N + 4), 7.0, device=dev)
-            assert ops._partial(lin, c, sp, x2, P[:, :, :N], M) == 0
+            P = torch.full((sp, M + 128, N + 4), 7.0, device=dev)
+            assert ops._partial(lin, c, sp, x2, P[:, :M, :N], M) == 0
             out.append(P.cpu())
         assert torch.equal(out[0], out[1])
+        assert torch.all(out[1][:, M:] == 7.0) and torch.all(out[1][:, :, N:] == 7.0)
 
 
 def test_mid_tiles_take_what_the_config_took(dev):
