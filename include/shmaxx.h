@@ -61,8 +61,9 @@ int mx_gemm_bf16_partial(hipStream_t st, int cfg, int splits, const uint16_t* A,
 int mx_gemm_reduce(hipStream_t st, const float* P, int nsplit, long p_split, long ldp, const float* bias,
                    const uint16_t* R, long ldr, int r_rows, uint16_t* C, long ldc, int M, int N, int act,
                    int act_ncols);
-/* mx_gemm_bf16 and mx_gemm_reduce with the activation (act 1 or 2; act 3 is refused) on columns >= act_from only: one
- * product over the fused [qkv | fc1] rows of the parallel text block (md2fast.py:173-198) with fc1's GELU. */
+/* mx_gemm_bf16 and mx_gemm_reduce with the activation (act 1 or 2; act 3 is refused) on columns >= act_from only
+ * (act_from % 4 == 0, else MX_ESHAPE): one product over the fused [qkv | fc1] rows of the parallel text block
+ * (md2fast.py:173-198) with fc1's GELU. */
 int mx_gemm_bf16_act_from(hipStream_t st, int cfg, int splits, const uint16_t* A, long lda, const uint16_t* W, long ldw,
                           const float* bias, const uint16_t* R, long ldr, int r_rows, uint16_t* C, long ldc, int M,
                           int N, int K, int Kw, int act, int act_from, float* ws, long ws_elems, int* cnt, long n_cnt);

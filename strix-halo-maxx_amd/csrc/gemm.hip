@@ -1277,12 +1277,13 @@ extern "C" int mx_gemm_bf16(hipStream_t st, int cfg, int splits, const uint16_t*
 }
 
 // The same with the activation on columns >= act_from only (act 1, 2): the GELU of fc1's columns in one product over the
-// fused [qkv | fc1] rows.
+// fused [qkv | fc1] rows. act_from % 4 == 0: the epilogue decides per group of 4 columns.
 extern "C" int mx_gemm_bf16_act_from(hipStream_t st, int cfg, int splits, const uint16_t* A, long lda,
                                      const uint16_t* W, long ldw, const float* bias, const uint16_t* R, long ldr,
                                      int r_rows, uint16_t* C, long ldc, int M, int N, int K, int Kw, int act,
                                      int act_from, float* ws, long ws_elems, int* cnt, long n_cnt) {
   if (act_from < 0 || act == 3) return MX_EBADCFG;
+  if (act_from % 4) return MX_ESHAPE;
   return gemm_bf16(st, cfg, splits, A, lda, W, ldw, bias, R, ldr, r_rows, C, ldc, M, N, K, Kw, act, -act_from, ws,
                    ws_elems, cnt, n_cnt);
 }
@@ -1396,6 +1397,7 @@ extern "C" int mx_gemm_reduce_act_from(hipStream_t st, const float* P, int nspli
                                        const float* bias, const uint16_t* R, long ldr, int r_rows, uint16_t* C,
                                        long ldc, int M, int N, int act, int act_from) {
   if (act_from < 0 || act == 3) return MX_EBADCFG;
+  if (act_from % 4) return MX_ESHAPE;
   return gemm_reduce(st, P, nsplit, p_split, ldp, bias, R, ldr, r_rows, C, ldc, M, N, act, -act_from);
 }
 

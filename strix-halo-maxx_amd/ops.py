@@ -162,8 +162,8 @@ class MxLin:
 
     def __call__(self, x, gelu=False, res=None, pre=None, act=None, out=None, act_cols=0, act_from=0):
         """act: None / "tanh" / "erf" / "glu" (gated GELU on interleaved (gate, up) weight rows: output width N / 2);
-        act_cols > 0 limits the activation to output columns < act_cols, act_from > 0 to columns >= act_from (not both,
-        and not with "glu")."""
+        act_cols > 0 limits the activation to output columns < act_cols, act_from > 0 to columns >= act_from (a
+        multiple of 4; not both, and not with "glu")."""
         if act_from and (act_cols > 0 or act == "glu"):
             raise ValueError("act_from goes with neither act_cols nor glu")
         a = ACT[act if act is not None else gelu]

@@ -78,6 +78,16 @@ def test_gemm_entry_point_refuses_before_launch():
     assert rc == -2
 
 
+@pytest.mark.parametrize("act_from,act,rc", [(5, 1, -2), (2, 2, -2), (4303, 1, -2), (-4, 1, -1), (4, 3, -1)])
+def test_act_from_refused_before_launch(act_from, act, rc):
+    """The epilogue decides per group of 4 columns: a start inside a group would leave columns without the activation."""
+    lib = _lib.load()
+    assert lib.mx_gemm_bf16_act_from(None, 7, 1, A16, 1152, A16, 1152, A16, None, 0, 0, A16, 4304, 729, 4304, 1152, 1152,
+                                     act, act_from, None, 0, None, 0) == rc
+    assert lib.mx_gemm_reduce_act_from(None, A16, 2, 729 * 4304, 4304, A16, None, 0, 0, A16, 4304, 729, 4304, act,
+                                       act_from) == rc
+
+
 def test_gemm_pick_is_a_valid_config():
     lib = _lib.load()
     for M, N, K in [(729, 3456, 1152), (729, 1152, 4352), (186624, 4304, 1152), (1, 6144, 2048)]:

@@ -38,3 +38,7 @@ def test_act_from_refusals(dev):
         lin(x, act="tanh", act_from=8, act_cols=4)
     with pytest.raises(_lib.MxError):
         lin(x, act="tanh", act_from=-4)
+    for cfg in ((7, 1), (22, -1)):
+        lin.cfgs[8] = cfg
+        with pytest.raises(_lib.MxError):
+            lin(x, act="tanh", act_from=5)
