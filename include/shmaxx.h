@@ -292,7 +292,9 @@ int mx_decode_step_mk_i8(hipStream_t st, const void* layers, int nl, int ctx, co
                          const uint16_t* lnf_b, const uint16_t* wlm, const float* blm, int V, const uint16_t* wte,
                          const float* cs, float eps, float scale, uint16_t* x, int* state, int pos_base, int* tokens,
                          int cap, uint16_t* logits, uint64_t* ll, uint32_t* ep);
-/* The same two steps for caches of up to 2048 positions (ctx <= 2048, else MX_ESHAPE). */
+/* The same two steps for caches of up to 2048 positions (ctx <= 2048, else MX_ESHAPE). Like them only for a caller that
+ * checks ep[1] or has the device to itself: two such steps at once (two streams, two processes) may each hold CUs that
+ * the other waits for, and time out. */
 int mx_decode_step_mk_long(hipStream_t st, const void* layers, int nl, int ctx, const uint16_t* lnf_g,
                            const uint16_t* lnf_b, const uint16_t* wlm, const float* blm, int V, const uint16_t* wte,
                            const float* cs, float eps, float scale, uint16_t* x, int* state, int pos_base, int* tokens,

@@ -130,13 +130,18 @@ class TextDecoder:
         # one launch per decode step (mx_decode_step_mk, or mx_decode_step_mk_i8 for the W8A8 Linears) where its
         # shapes hold: the 2048-wide, 32 x 64-head, 8192-MLP model, a cache of at most 2048 positions (past 1024 its
         # _long form, whose attention takes the keys in two passes), one attention split, and a device with a CU for
-        # each of its workgroups; the per-layer kernels above otherwise (use_mk = False selects them too)
+        # each of its workgroups; the per-layer kernels above otherwise (use_mk = False selects them too).
+        # Its 256 workgroups wait for each other: where two such steps run at once (two decoders on two streams, another
+        # process), neither may get all its workgroups resident, and after 50 ms the tokens are undefined and mk_error()
+        # is set, which only generate() looks at. Caches past 1024 positions therefore keep the per-layer kernels, which
+        # wait for nobody, unless the program sets use_mk = True for a decoder that has the device to itself (before
+        # capture_step; 4 W8A8 layers at 1500 keys: 140 us a step per layer, 122 in one launch).
         self.mk_layers = self.mk_ll = self.mk_ep = None
         if (dev.type == "cuda" and attn_splits == 1 and (self.D, self.H, self.hd, c["ff"]) == (2048, 32, 64, 8192)
                 and ctx <= 2048 and self.V <= 65536
                 and torch.cuda.get_device_properties(dev).multi_processor_count >= lib.mx_decode_mk_grid()):
             self._init_mk()
-        self.use_mk = self.mk_layers is not None
+        self.use_mk = self.mk_layers is not None and ctx <= 1024
         self.mk_fallbacks = 0  # generations redone on the per-layer kernels after a one-launch step timed out
 
     def _init_mk(self):

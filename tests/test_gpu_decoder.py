@@ -485,7 +485,7 @@ def test_one_launch_step_past_1024_keys(dev, start, w8a8):
     up to the last cache row (2047). Tolerances as for the one-pass form: the two differ by fp32 summation orders
     (5e-3), or by an int8 step of the LayerNorm's output (2e-2)."""
     dec = mt.TextDecoder(S.text_weights(2, layers=2), ctx=2048, w8a8=w8a8)
-    assert dec.use_mk
+    assert dec.mk_layers is not None
     img = S.activations(7, (729, 2048), "img").to(dev)
     prompt = S.prompt_ids(8, start - 730)
     out = {}
@@ -501,6 +501,43 @@ def test_one_launch_step_past_1024_keys(dev, start, w8a8):
         out[mk] = (dec.tokens[:7].cpu().tolist(), lg, dec.xd[0].cpu().clone())
     assert dec.mk_error() == 0 and dec.mk_fallbacks == 0 and dec.state.cpu().tolist() == [7, start + 6]
     compare_free_running(out, 2e-2 if w8a8 else 5e-3)
+
+
+@pytest.mark.parametrize("ctx,one_launch", [(1024, True), (1025, False), (2048, False)])
+def test_long_caches_decode_on_the_per_layer_kernels(dev, ctx, one_launch):
+    """decode_step and capture_step never look at mk_error(): past 1024 positions the step that can time out beside
+    another one is taken only where the program asks for it (use_mk = True)."""
+    assert mt.TextDecoder(S.text_weights(2, layers=1), ctx=ctx).use_mk is one_launch
+
+
+def test_two_long_decoders_on_two_streams(dev):
+    """Two decoders with 2048-entry caches, steps interleaved on two streams, give the tokens and logits that each gives
+    alone, bit for bit (fixed kernels, no cross-workgroup waits)."""
+    decs = [mt.TextDecoder(S.text_weights(2 + i, layers=2), ctx=2048) for i in range(2)]
+    imgs = [S.activations(7 + i, (729, 2048), "img").to(dev) for i in range(2)]
+    alone = []
+    for d, img in zip(decs, imgs):
+        d.prefill(img, S.prompt_ids(8, 400))
+        d.start_decode()
+        lg = []
+        for _ in range(8):
+            d.decode_step(logits=True)
+            lg.append(d.logits.cpu().clone())
+        alone.append((d.tokens[:9].cpu().tolist(), lg))
+    for d, img in zip(decs, imgs):
+        d.prefill(img, S.prompt_ids(8, 400))
+        d.start_decode()
+    torch.cuda.synchronize()
+    streams, got = [torch.cuda.Stream() for _ in decs], [[], []]
+    for _ in range(8):
+        for i, d in enumerate(decs):
+            with torch.cuda.stream(streams[i]):
+                d.decode_step(logits=True)
+                got[i].append(d.logits.clone())
+    torch.cuda.synchronize()
+    for i, d in enumerate(decs):
+        assert d.tokens[:9].cpu().tolist() == alone[i][0] and d.mk_error() == 0
+        assert all(torch.equal(a, b.cpu()) for a, b in zip(alone[i][1], got[i]))
 
 
 YES, NO = [11, 222, 3333, 44444], [55, 666, 7777, 50000]
