@@ -963,6 +963,9 @@ struct Cfg { int bm, bn, stages, per_cu, kind, waves, kh = 1; };
 // kind 0: LDS-shared tile split over the waves; kind 1: wave-split K (each wave the whole tile, a quarter of K).
 // Both stage operands through a `stages`-deep LDS ring.
 // per_cu: workgroups that fit one CU at once (LDS- or register-limited)
+// The int8 GEMM runs every one of these as it stands. In bf16 configs 15, 17, 19, 25 and 27 keep only their tile sizes
+// and their split rules (mx_gemm_check, psum_ok): gemm_big.hip (15, 25: persistent, 4 waves) and gemm_mid.hip (17, 19, 27,
+// and 5 for partials: 4 waves, one k chain) take them.
 constexpr Cfg kCfgs[] = {{128, 128, 4, 1, 0, 4}, {64, 128, 4, 1, 0, 4}, {128, 64, 4, 1, 0, 4}, {64, 64, 4, 2, 0, 4},
                          {256, 128, 3, 1, 0, 4}, {128, 256, 3, 1, 0, 4}, {64, 64, 3, 3, 0, 4}, {128, 128, 2, 2, 0, 4},
                          {64, 64, 4, 2, 1, 4},   {64, 128, 4, 1, 1, 4},  {128, 64, 4, 1, 1, 4}, {64, 64, 3, 3, 1, 4},
@@ -1212,7 +1215,8 @@ int gemm_bf16(hipStream_t st, int cfg, int splits, const uint16_t* A, long lda, 
   const int rc = mx_gemm_check(cfg, splits, A, lda, W, ldw, bias, R, ldr, C, ldc, M, N, K, Kw, act, ws, ws_elems, cnt, n_cnt);
   if (rc) return rc;
   hipError_t e;
-#define L_(BM, BN, S) launch<BM, BN, 2, 2, S>(st, splits, A, lda, W, ldw, bias, R, ldr, r_rows, C, ldc, M, N, K, Kw, act, act_ncols, ws, cnt)
+#define GEMM_ARGS_ st, splits, A, lda, W, ldw, bias, R, ldr, r_rows, C, ldc, M, N, K, Kw, act, act_ncols, ws, cnt
+#define L_(BM, BN, S) launch<BM, BN, 2, 2, S>(GEMM_ARGS_)
   switch (cfg) {
     case 0: e = L_(128, 128, 4); break;
     case 1: e = L_(64, 128, 4); break;
@@ -1222,20 +1226,41 @@ int gemm_bf16(hipStream_t st, int cfg, int splits, const uint16_t* A, long lda, 
     case 5: e = L_(128, 256, 3); break;
     case 6: e = L_(64, 64, 3); break;
     case 7: e = L_(128, 128, 2); break;
-    case 23: e = launch<96, 128, 1, 4, 4>(st, splits, A, lda, W, ldw, bias, R, ldr, r_rows, C, ldc, M, N, K, Kw, act, act_ncols, ws, cnt); break;
+    case 23: e = launch<96, 128, 1, 4, 4>(GEMM_ARGS_); break;
     case 15: case 25: {
-      // the persistent tiles; what they do not take (rows of C or R not in whole 16-byte chunks, K <= 192) runs on the
-      // 128 x 128 tile of config 7: the same bits
       const BigGemm g{A, lda, W, ldw, bias, R, ldr, r_rows, C, ldc, M, N, K, Kw, act_ncols};
-      e = gemm_big_fits(act, g) ? launch_gemm_big(st, kCfgs[cfg].bn, act, g) : L_(128, 128, 2);
+      // What the persistent tiles do not take (rows of C or R not in whole 16-byte chunks, K <= 192) runs on the 8-wave
+      // tile of the same size where that fills the chip, else on config 7's: the same bits. us, 8-wave / config 7, rows
+      // of 8 bytes: 40960 x 4300 x 1152 494 / 545, 9472 x 1156 x 4352 103 / 117, 8192 x 1028 x 768 30.8 / 30.5 (10 M
+      // outputs), 8192 x 772 x 1152 37.0 / 26.1; 256 x 192: 9472 x 3460 x 1152 96 / 102, 8192 x 1028 x 2048 49 / 60
+      // (9.4 M), 8192 x 772 x 2048 44 / 38.
+      const bool fills = tiles_of(cfg, M, N) * kCfgs[cfg].bm * kCfgs[cfg].bn >= 9L << 20;
+      if (gemm_big_fits(act, g))
+        e = launch_gemm_big(st, kCfgs[cfg].bn, act, g);
+      else if (!fills)
+        e = L_(128, 128, 2);
+      else
+        e = cfg == 15 ? launch<256, 256, 2, 4, 2>(GEMM_ARGS_) : launch<256, 192, 4, 2, 2>(GEMM_ARGS_);
       break;
     }
-    case 16: e = launch<256, 128, 4, 2, 3>(st, splits, A, lda, W, ldw, bias, R, ldr, r_rows, C, ldc, M, N, K, Kw, act, act_ncols, ws, cnt); break;
+    case 16: e = launch<256, 128, 4, 2, 3>(GEMM_ARGS_); break;
     case 17: case 19: case 27: {
-      // the one-tile-per-CU tiles; what they do not take (rows of C or R not in whole 16-byte chunks) runs on the
-      // 128 x 128 tile of config 7: the same bits
       const BigGemm g{A, lda, W, ldw, bias, R, ldr, r_rows, C, ldc, M, N, K, Kw, act_ncols};
-      e = gemm_mid_fits(act, g) ? launch_gemm_mid(st, kCfgs[cfg].bn, act, g) : L_(128, 128, 2);
+      // What the one-tile-per-CU tiles do not take (rows of C or R not in whole 16-byte chunks): config 7's tile, two
+      // workgroups per CU; the 4-stage ring of config 0 where one per CU is all there is and K is deep, and 128 x 192
+      // where its grid is one round that nearly fills the chip. All one k chain: the same bits. us, that tile / config
+      // 7's, rows of 8 bytes: config 0's 768 x 1156 x 4352 37.7 / 47.7, 600 x 6148 x 2048 24.6 / 26.7, 768 x 4300 x 1152
+      // 18.8 / 18.3; 128 x 192: 768 x 6148 x 2048 30.6 / 33.9 (198 tiles), 2048 x 2308 x 1152 21.8 / 23.3 (208), 640 x
+      // 6148 x 2048 30.1 / 28.2 (165), 8192 x 772 x 1152 37.6 / 26.1 (320).
+      const long t = tiles_of(cfg, M, N);
+      if (gemm_mid_fits(act, g))
+        e = launch_gemm_mid(st, kCfgs[cfg].bn, act, g);
+      else if (cfg == 19 && t <= 256 && Kw >= 2048)
+        e = L_(128, 128, 4);
+      else if (cfg == 27 && t >= 176 && t <= 256)
+        e = launch<128, 192, 4, 2, 3>(GEMM_ARGS_);
+      else
+        e = L_(128, 128, 2);
       break;
     }
     case 18: e = L_(256, 256, 2); break;
@@ -1256,6 +1281,7 @@ int gemm_bf16(hipStream_t st, int cfg, int splits, const uint16_t* A, long lda, 
     default: return MX_EBADCFG;
   }
 #undef L_
+#undef GEMM_ARGS_
 #undef W_
 #undef H_
   return e == hipSuccess ? MX_OK : MX_ELAUNCH;

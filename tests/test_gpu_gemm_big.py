@@ -51,3 +51,21 @@ def test_big_tiles_take_what_the_config_took(dev):
             lin(x, out=y[:, :N])
             out.append(y.cpu())
         assert torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
+
+
+@pytest.mark.parametrize("M,N,cfg", [(40900, 132, 15), (49100, 132, 25), (8200, 1036, 15), (8200, 1036, 25)])
+def test_big_tiles_unaligned_large_grids(dev, M, N, cfg):
+    """The same calls where the 8-wave tile of the config's size fills the chip (from 9 M outputs of whole tiles)."""
+    g = torch.Generator().manual_seed(M)
+    x = torch.randn(M, 136, generator=g).to(BF).to(dev)
+    lin = ops.MxLin((torch.randn(N, 136, generator=g) * 0.02).to(BF), torch.randn(N, generator=g) * 0.02)
+    r = torch.randn(M, N, generator=g).to(BF).to(dev)
+    for kw in (dict(), dict(gelu=True), dict(res=r)):
+        out = []
+        for c in (7, cfg):
+            lin.cfgs[M] = (c, 1)
+            y = torch.full((M + 256, N + 8), 7.0, device=dev, dtype=BF)
+            lin(x, out=y[:M, :N], **kw)
+            out.append(y)
+        print(f"unaligned cfg={cfg} {M}x{N} {[k for k in kw]}", flush=True)
+        assert torch.equal(out[0], out[1]) and torch.all(out[1][M:] == 7.0) and torch.all(out[1][:, N:] == 7.0)

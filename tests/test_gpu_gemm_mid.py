@@ -72,3 +72,21 @@ def test_mid_tiles_take_what_the_config_took(dev):
             lin(x, out=y[:, :N])
             out.append(y.cpu())
         assert all(torch.equal(out[0], o) for o in out[1:])
+
+
+# (config, M, N, K): config 0's tile (one workgroup per CU, deep K), the 128 x 192 tile (176 .. 256 of them)
+@pytest.mark.parametrize("cfg,M,N,K", [(19, 130, 132, 2056), (19, 300, 1220, 2504), (27, 1700, 2308, 200), (27, 32700, 132, 72)])
+def test_mid_tiles_unaligned_grids(dev, cfg, M, N, K):
+    g = torch.Generator().manual_seed(M)
+    x = torch.randn(M, K, generator=g).to(BF).to(dev)
+    lin = ops.MxLin((torch.randn(N, K, generator=g) * 0.02).to(BF), torch.randn(N, generator=g) * 0.02)
+    r = torch.randn(M, N, generator=g).to(BF).to(dev)
+    for kw in (dict(), dict(gelu=True), dict(res=r)):
+        out = []
+        for c in (7, cfg):
+            lin.cfgs[M] = (c, 1)
+            y = torch.full((M + 128, N + 8), 7.0, device=dev, dtype=BF)
+            lin(x, out=y[:M, :N], **kw)
+            out.append(y)
+        print(f"unaligned cfg={cfg} {M}x{N}x{K} {[k for k in kw]}", flush=True)
+        assert torch.equal(out[0], out[1]) and torch.all(out[1][M:] == 7.0) and torch.all(out[1][:, N:] == 7.0)
