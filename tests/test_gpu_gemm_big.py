@@ -11,7 +11,7 @@ BF = torch.bfloat16
 
 
 # one row; the last tile a row / 8 columns wide; an odd number of k-steps (904 = 14.1, 320 = 5); the fewest steps (256);
-# whole tiles; more than one tile per CU with an odd last one (300 tiles of either width)
+# whole tiles; more than one tile per CU with an odd last one (300 tiles of 256 columns, 600 of 192)
 @pytest.mark.parametrize("M,N,K", [(1, 16, 256), (257, 272, 904), (300, 200, 320), (512, 768, 1152), (76699, 208, 256)])
 @pytest.mark.parametrize("cfg", [15, 25])
 def test_big_tiles_equal_the_small_one(dev, cfg, M, N, K):
@@ -69,3 +69,26 @@ def test_big_tiles_unaligned_large_grids(dev, M, N, cfg):
             out.append(y)
         print(f"unaligned cfg={cfg} {M}x{N} {[k for k in kw]}", flush=True)
         assert torch.equal(out[0], out[1]) and torch.all(out[1][M:] == 7.0) and torch.all(out[1][:, N:] == 7.0)
+
+
+# 313 row tiles (the last of 129 rows) x 5 column tiles of 256 or 7 of 192 (the last of 144 / 16 columns): 6 to 9 tiles per
+# workgroup of 256 CUs, so the bias rows' ring of 4 comes round and every tile's loads run into the next one's; 5 steps of
+# 64 (the odd step is followed by one of zeros) and 6
+@pytest.mark.parametrize("K", [320, 384])
+@pytest.mark.parametrize("cfg", [15, 25])
+def test_big_tiles_many_per_workgroup(dev, cfg, K):
+    M, N = 80001, 1168
+    g = torch.Generator(device=dev).manual_seed(K)
+    x = torch.randn(M, K, generator=g, device=dev).to(BF)
+    lin = ops.MxLin((torch.randn(N, K, generator=g, device=dev) * 0.02).to(BF), torch.randn(N, generator=g, device=dev))
+    r = torch.randn(M, N, generator=g, device=dev).to(BF)
+    for kw in (dict(), dict(gelu=True), dict(res=r), dict(act="glu")):
+        No = N // 2 if kw.get("act") == "glu" else N
+        out = []
+        for c in (7, cfg):
+            lin.cfgs[M] = (c, 1)
+            y = torch.full((M + 256, No + 8), 7.0, device=dev, dtype=BF)
+            lin(x, out=y[:M, :No], **kw)
+            out.append(y)
+        print(f"big cfg={cfg} {M}x{N}x{K} {[k for k in kw]}", flush=True)
+        assert torch.equal(out[0], out[1]) and torch.all(out[1][M:] == 7.0) and torch.all(out[1][:, No:] == 7.0), kw
