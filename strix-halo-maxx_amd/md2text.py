@@ -52,9 +52,9 @@ class TextDecoder:
         self.blocks = []
         for i in range(n):
             p = f"blocks.{i}."
-            # [Wqkv | Wfc1] stored once, fused: the decode GEMV streams both in one pass; the prefill GEMMs use row
-            # slices of the same storage (int8 with per-row scales in the W8A8 form: a row's scale is its own, so the
-            # fused quantisation equals quantising qkv and fc1 separately)
+            # [Wqkv | Wfc1] stored once, fused: the decode GEMV and the bf16 prefill product stream both in one pass; the
+            # W8A8 prefill and other Linear classes use row slices of the same storage (int8 with per-row scales in the
+            # W8A8 form: a row's scale is its own, so the fused quantisation equals quantising qkv and fc1 separately)
             wqf = torch.cat([weights[p + "attn.qkv.weight"], weights[p + "mlp.fc1.weight"]]).to(dev, BF).contiguous()
             bqf = torch.cat([weights[p + "attn.qkv.bias"], weights[p + "mlp.fc1.bias"]]).to(dev, torch.float32).contiguous()
             nqkv = weights[p + "attn.qkv.weight"].shape[0]
@@ -69,12 +69,14 @@ class TextDecoder:
                 blk["wp"], blk["swp"] = blk["proj"].wq, blk["proj"].sw
                 blk["w2"], blk["sw2"] = blk["fc2"].wq, blk["fc2"].sw
             else:
-                blk.update(wqf=wqf, qkv=lin_cls(wqf[:nqkv], bqf[:nqkv], BF), fc1=lin_cls(wqf[nqkv:], bqf[nqkv:], BF),
+                blk.update(wqf=wqf,
                            proj=lin_cls(weights[p + "attn.proj.weight"], weights[p + "attn.proj.bias"], BF),
                            fc2=lin_cls(weights[p + "mlp.fc2.weight"], weights[p + "mlp.fc2.bias"], BF))
                 blk["wp"], blk["w2"] = blk["proj"].w, blk["fc2"].w
                 if lin_cls is ops.MxLin:
                     blk["qf"] = ops.MxLin(wqf, bqf, BF, dev)  # the same storage
+                else:
+                    blk.update(qkv=lin_cls(wqf[:nqkv], bqf[:nqkv], BF), fc1=lin_cls(wqf[nqkv:], bqf[nqkv:], BF))
             blk["bp"], blk["b2"] = f32(p + "attn.proj.bias"), f32(p + "mlp.fc2.bias")
             self.blocks.append(blk)
         self.post_ln = (g("post_ln.weight"), g("post_ln.bias"))
@@ -188,8 +190,10 @@ class TextDecoder:
             pre = b["qkv"].quant(h) if self.w8a8 else None
             if "qf" in b:
                 # qkv and fc1 (its GELU on its own columns) as one product over the fused rows: a launch less, and a
-                # grid of 14336 columns fills the device (us, two products -> one: 32 rows 24.5 -> 17.2, 256 40.0 ->
-                # 28.2, 730 60.4 -> 45.9, 794 60.3 -> 55.9)
+                # grid of 14336 columns fills the device (us, two products -> one, cold weights: 32 rows 23.5 -> 16.4,
+                # 256 36.1 -> 27.3, 730 58.4 -> 43.6, 794 56.3 -> 55.7, 1100 74.7 -> 72.0, 1409 89.6 -> 86.5). Where two
+                # grids of whole rounds add up to fewer than one's, two products would be faster: 1216 74.8 against
+                # 79.8, from 1537 rows on 95.0 against 102.3.
                 y = b["qf"](h, act="tanh", act_from=b["nq"])
                 qkv, f = y[:, :b["nq"]], y[:, b["nq"]:]
             else:

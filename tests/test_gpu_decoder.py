@@ -540,6 +540,22 @@ def test_two_long_decoders_on_two_streams(dev):
         assert all(torch.equal(a, b.cpu()) for a, b in zip(alone[i][1], got[i]))
 
 
+def test_prefill_holds_the_linears_it_runs(dev):
+    """bf16 MxLin blocks hold the fused [qkv | fc1] Linear and no row slices of it; another Linear class holds the slices.
+    Both prefill the same: the two differ by fp32 summation orders of the products (5e-3, as between decode paths)."""
+    class Other(ops.MxLin):
+        pass
+    w = S.text_weights(2, layers=2)
+    a, b = mt.TextDecoder(w, ctx=1024), mt.TextDecoder(w, lin_cls=Other, ctx=1024)
+    assert all("qf" in x and "qkv" not in x and "fc1" not in x for x in a.blocks)
+    assert all("qf" not in x and "qkv" in x and "fc1" in x for x in b.blocks)
+    img, ids = S.activations(7, (100, 2048), "img").to(dev), S.prompt_ids(8, 20)
+    x, y = a.prefill(img, ids).float(), b.prefill(img, ids).float()
+    assert float((x - y).norm() / y.norm()) < 5e-3
+    la, lb = a.logits.float(), b.logits.float()
+    assert float((la - lb).norm() / lb.norm()) < 2e-2
+
+
 YES, NO = [11, 222, 3333, 44444], [55, 666, 7777, 50000]
 
 
