@@ -864,7 +864,12 @@ def large_batch_block_ops(vt, imgs):
             "fc2": (2 * M * F * D, 2 * (M * F + D * F + 2 * M * D), lambda: b["fc2"](f, res=x1, out=y))}
 
 
-PROBES = ("tower_b256", "trecvit", "scan", "decode_w8a8", "prefill")
+PROBES = ("tower_b256", "trecvit", "scan", "decode_w8a8", "prefill", "gemm")
+
+# the gemm probe: (tile config, M, N, K, activation, splits of raw partials or 0)
+GEMM_PROBE = ((15, 8192, 8192, 8192, None, 0), (15, 186624, 3456, 1152, None, 0), (15, 186624, 4304, 1152, "tanh", 0),
+              (25, 186624, 1152, 4304, None, 0), (27, 794, 6144, 2048, None, 0), (17, 794, 8192, 2048, "tanh", 0),
+              (19, 729, 4304, 1152, "tanh", 0), (19, 729, 1152, 4304, None, 4))
 
 
 def _probe_classes(workload):
@@ -942,6 +947,23 @@ def _probe_classes(workload):
         fl = 2 * L * (3 * D * D + D * D + 2 * D * F_) * n + 4 * L * D * (P * P + (n - P) * n)
         return ("moondream2 text prefill, 24 layers, 730 prefix + 64 prompt rows in one pass, eager launches",
                 [("prefill", lambda: dec.prefill(img, prompt), None, fl)])
+    if workload == "gemm":
+        import strix_halo_maxx_amd.ops as ops
+        g = torch.Generator(device=dev).manual_seed(4)
+        rnd = lambda *shape: torch.randn(*shape, device=dev, generator=g).to(torch.bfloat16)
+        classes = []
+        for cfg, M, N, K, act, sp in GEMM_PROBE:
+            lin, x = ops.MxLin(rnd(N, K) * 0.02, torch.zeros(N)), rnd(M, K)
+            if sp:
+                P = torch.empty(sp, M, N, device=dev)
+                fn = lambda lin=lin, x=x, P=P, c=cfg, sp=sp: ops._partial(lin, c, sp, x, P, P.shape[1])
+            else:
+                lin.cfgs[M] = (cfg, 1)
+                fn = lambda lin=lin, x=x, act=act, y=torch.empty(M, N, device=dev, dtype=torch.bfloat16): lin(x, act=act, out=y)
+            fn()
+            classes.append((f"{cfg}: {M} x {N} x {K}" + (f", {sp} splits" if sp else "") + (", GELU" if act else ""), fn,
+                            2 * (M * K + N * K) + (4 * sp if sp else 2) * M * N, 2 * M * N * K))
+        return "the persistent and the software-pipelined GEMM tiles (config: M x N x K), eager launches", classes
     raise ValueError(f"unknown probe {workload}; one of {PROBES}")
 
 
@@ -991,7 +1013,7 @@ def summarize_probe(workload, paths, reps=3):
     """Markdown summary of rocprofv3 --pmc passes (one CSV each) over `bench.py --probe WORKLOAD`: per class, per
     (kernel, grid): dispatches per call, HBM traffic per dispatch from FETCH_SIZE / WRITE_SIZE (scaled by what the
     counters read for the 256 MiB calibration copies), and whichever of MfmaUtil, the waiting / issue fractions of
-    wave time, LDS bank conflicts and the L2 hit rate the CSVs hold."""
+    wave time, LDS bank conflicts, the L2 hit rate and the vector L1s' read requests the CSVs hold."""
     title, classes = _probe_classes(workload)
     vals = {}
     for p in paths:
@@ -1031,7 +1053,7 @@ def summarize_probe(workload, paths, reps=3):
                 rd, wr = stat("FETCH_SIZE") * 1024 * cal["FETCH_SIZE"], stat("WRITE_SIZE") * 1024 * cal["WRITE_SIZE"]
                 e.update(read_bytes=int(rd), write_bytes=int(wr))
             for c in ("MfmaUtil", "SQ_WAIT_ANY", "SQ_WAVE_CYCLES", "SQ_WAIT_INST_ANY", "SQ_ACTIVE_INST_VALU",
-                      "SQ_ACTIVE_INST_LDS", "SQ_LDS_BANK_CONFLICT", "TCC_HIT_sum", "TCC_MISS_sum"):
+                      "SQ_ACTIVE_INST_LDS", "SQ_LDS_BANK_CONFLICT", "TCC_HIT_sum", "TCC_MISS_sum", "TCP_TCC_READ_REQ_sum"):
                 if c in segs:
                     e[c] = stat(c)
             if algo and len(order) == 1:
@@ -1058,6 +1080,8 @@ def summarize_probe(workload, paths, reps=3):
         cols.append(("LDS bank-conflict cycles", lambda e: f"{e['SQ_LDS_BANK_CONFLICT']:,.0f}"))
     if "TCC_HIT_sum" in have and "TCC_MISS_sum" in have:
         cols.append(("L2 hit rate", lambda e: f"{e['TCC_HIT_sum'] / max(1.0, e['TCC_HIT_sum'] + e['TCC_MISS_sum']):.2f}"))
+    if "TCP_TCC_READ_REQ_sum" in have:
+        cols.append(("read requests to the L2s", lambda e: f"{e['TCP_TCC_READ_REQ_sum']:.3g}"))
     lines = ["| class | kernel | grid threads | " + " | ".join(c for c, _ in cols) + " |",
              "|" + "---|" * (len(cols) + 3)]
     for e in blob["kernels"]:
