@@ -147,9 +147,21 @@ def tune_generic(log):
         del vt
         torch.cuda.empty_cache()
         dec = md2text.TextDecoder(S.text_weights(0), device=dev, ctx=1024, yes_ids=(11, 222), no_ids=(55, 666))
-        dec.prefill(S.activations(3, (729, 2048), "img").to(dev), S.prompt_ids(4, 64))
+        img = S.activations(3, (729, 2048), "img").to(dev)
+        dec.prefill(img, S.prompt_ids(4, 64))
+        dec.encode(img)                                     # the image prefix alone: 730 rows
         dec.set_questions([S.prompt_ids(4, 32).tolist()])   # the yes/no query: 32 rows
         dec.query()
+        # one Linear at a time, for programs that run the text layers' products separately (qkv and fc1 as two: the
+        # reference's own forward through refbind), prompts of 64 rows included
+        b = dec.blocks[0]
+        lins = [ops.MxLin(b["wqf"][:b["nq"]], b["bqf"][:b["nq"]]), ops.MxLin(b["wqf"][b["nq"]:], b["bqf"][b["nq"]:]), b["qf"],
+                b["proj"], b["fc2"]]
+        for M in (32, 64, 730, 794):
+            for lin in lins:
+                lin(torch.randn(M, lin.K, device=dev).to(torch.bfloat16))
+        for M in (730, 794):  # a partial pick is what has fc2's reduction fused with the next LayerNorm
+            b["fc2"].partial(torch.randn(M, b["fc2"].K, device=dev).to(torch.bfloat16))
         torch.cuda.synchronize()
         log("text prefill and query tuned")
         del dec
@@ -162,6 +174,8 @@ def tune_generic(log):
         m.reset()
         m.clip_state(16)
         m.forward_clip(fr, qf)
+        for N, K in ((768, 768), (768, 3072)):  # the residual Linears of a frame on their own, without the fused norm
+            ops.MxLin(torch.randn(N, K, device=dev) * 0.02, None)(torch.randn(1280, K, device=dev).to(torch.bfloat16))
         torch.cuda.synchronize()
         log("trecvit tuned")
     fused = {k: v for k, v in ops._TUNED.items() if k not in before}
@@ -183,7 +197,7 @@ def main():
     part.update(p1)
     key = lambda k: ",".join(str(v) for v in k)
     lines = ["{", ' "note": "MI355X (gfx950) GEMM tile table: (M, N, Kw) -> (tile config, splits: > 0 in-kernel, -S = S '
-                  'raw partials + mx_gemm_reduce); written by python -m strix_halo_maxx_amd.tune",']
+                  'raw partials + mx_gemm_reduce); picks of python -m strix_halo_maxx_amd.tune",']
     for name, d, last in (("fused", fused, False), ("partial", part, True)):
         items = [f'  "{key(k)}": [{v[0]}, {v[1]}]' for k, v in sorted(d.items())]
         lines += [f' "{name}": {{', ",\n".join(items), " }" + ("" if last else ",")]
