@@ -23,7 +23,7 @@
 //     Each compute wave streams A and B through a ring of MK_NB 4 KB units (the next unit issued as soon as one is
 //     reduced, across phase and layer boundaries).
 //   * attention workgroups 224 .. 255, one per head: the compute waves load the head's K cache rows 0 .. pos - 1
-//     into registers and its V rows into LDS (LDS-DMA), 8 keys per wave per round, 16 rounds (contexts up to 1024),
+//     into registers and its V rows into LDS (LDS-DMA), 8 keys per wave per round, 16 rounds (1024 keys; LONG: passes of 1024),
 //     as soon as the previous layer's attention is done; the exchange wave waits for the head's q / k / v, applies
 //     the rope (fp32, as rope.hip), and after the compute waves' one-pass softmax (merged in LDS) publishes the
 //     output and appends k / v at pos.
@@ -599,7 +599,8 @@ __global__ __launch_bounds__(MK_T) void decode_mk_kernel(MkArgs a) {
       // 1024 through the same registers and LDS rows (a wave reads only the rows it copied itself, so it refills them
       // without a barrier), K while the pass before it is weighted, V after it; the wave's maximum, sum and output are
       // rescaled from pass to pass. The second pass's V copy is waited for, about 3 us a layer: 4 W8A8 layers and the LM
-      // head take 114 us at 1000 keys, 127 at 1025, 128 at 1500, 131 at 2000; the per-layer kernels 132 / 136 / 147 / 148.
+      // head take 114 us at 1000 keys, 127 at 1025, 128 at 1500, 131 at 2000; the per-layer kernels 132 / 136 / 147 / 148
+      // (another box, 1500 keys: 122 and 140).
       const int sub = lane & 7, kg = lane >> 3;
       const uint32_t koff = (uint32_t)(wave * 8 + kg) * 128u + (uint32_t)sub * 16u;
       for (int l = 0; l < NL; l++) {

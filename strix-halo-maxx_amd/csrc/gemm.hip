@@ -1147,7 +1147,9 @@ extern "C" long mx_gemm_ws_counters(int cfg, int splits, int M, int N) {
 }
 
 // Default (cfg, splits) when the caller passes cfg < 0: minimise estimated time = rounds of workgroups over the
-// 256 CUs x per-tile time, with per-tile time ~ BM*BN*(k-steps)/efficiency. Returns cfg * 16 + splits.
+// 256 CUs x per-tile time, with per-tile time ~ BM*BN*(k-steps)/efficiency. Returns cfg * 16 + splits. The efficiencies of
+// 15, 17, 19, 25 and 27 are those of the 8-wave tiles that these were: the pick takes small tiles (8, 11, 12, 14, 3) at
+// every model shape and reaches neither the persistent nor the pipelined kernels; the table and the tuner (ops.MxLin) do.
 extern "C" int mx_gemm_pick(int M, int N, int Kw) {
   static const float eff[] = {1.0f, 0.78f, 0.78f, 0.6f, 1.1f, 1.1f, 0.6f, 0.9f, 1.0f, 1.0f, 1.0f, 1.0f,
                               1.0f, 1.0f, 1.0f, 1.3f, 1.1f, 1.1f, 1.4f, 1.1f, 0.9f, 0.9f, 0.7f, 0.9f,

@@ -1,5 +1,5 @@
 // bf16 GEMM for large grids: C[M,N] = epi(A[M,K] . W[N,K]^T + bias[N]), tiles of 256 x 256 or 256 x 192, with the operand
-// contract and the roundings of gemm.hip (and its k order: the same bits as its other tiles).
+// contract and the roundings of gemm.hip, every sum one fp32 chain in k order (the bits of its one-chain tiles).
 //
 // One persistent workgroup of 4 waves per CU, one wave per SIMD, each wave a 128 x (BN / 2) quarter of the tile in
 // 256 or 192 accumulator registers. What bounded the 8-wave tiles that this replaced (one tile per workgroup, a ring of
@@ -9,8 +9,8 @@
 //    one step to land in. Here the unit is a block of 64 rows (32 of each wave row): a step multiplies A block by A
 //    block, all of W's fragments in registers, so the blocks of a slot are read, freed and refilled one after another,
 //    at most one load instruction per two MFMAs, and a load has one and a half steps to land in. Rows stay 128 bytes in
-//    memory and in LDS: with 64-byte rows (32 columns, four slots) the L1 fetched every line twice (1.35e8 instead of
-//    6.7e7 requests to the L2 at 8192^3), which cost more than the longer ring gave.
+//    memory and in LDS: a copy with 64-byte rows (32 columns, four slots) made the L1 fetch every line twice (1.35e8
+//    instead of 6.7e7 requests to the L2 at 8192^3), which cost more than the longer ring gave.
 //  * The ramp at the start of a tile and the write-out at its end, a quarter of the time at K = 1152: the loads of the
 //    next tile's first steps are in flight through both, the sums start from the constant 0, and the results leave
 //    through a private 4 KB of LDS per wave in three overlapped stages without barriers.
@@ -19,14 +19,14 @@
 // buffer resources: one add per load, and rows past the edge need no clamping. For the same reason the activation
 // is not spread over the next tile's steps: 192 waiting values per lane and 10 instructions per value between the
 // MFMAs took longer than the write-out they would have hidden (qkv below: 1.35 ms).
-// Measured (us, before -> now; the 8-wave tile before, the better of both widths):
-//   186624 x 3456 x 1152           1460 -> 1255 (1184 TFLOP/s; MFMAs and LDS reads alone 935)
-//   186624 x 4304 x 1152, GELU     2011 -> 1771
-//   186624 x 1152 x 4304, residual 2068 -> 1709
-//   186624 x 1152 x 1152, residual  659 ->  507
-//   20480 x 6144 x 768, gated GELU  217 ->  192
-//   9477 x 3456 x 1152             84.9 -> 71.6
-//   8192 x 8192 x 8192              851 ->  770 (1427 TFLOP/s)
+// Measured (us, both on one box: the 8-wave tile before -> this one, each the better of both widths):
+//   186624 x 3456 x 1152           1495 -> 1319 (1127 TFLOP/s)
+//   186624 x 4304 x 1152, GELU     2034 -> 1842
+//   186624 x 1152 x 4304, residual 2092 -> 1756
+//   186624 x 1152 x 1152, residual  669 ->  522
+//   20480 x 6144 x 768, gated GELU  222 ->  196
+//   9477 x 3456 x 1152             89.5 -> 75.3
+//   8192 x 8192 x 8192              889 ->  807 (1363 TFLOP/s, MFMAs busy 75 % of the cycles)
 #include "gemm_out.h"
 
 namespace {

@@ -1,6 +1,8 @@
 // bf16 GEMM for grids of about one tile per CU: C[M,N] = epi(A[M,K] . W[N,K]^T + bias[N]) or raw fp32 split-K partials,
-// tiles of 128 x 128, 128 x 192 or 128 x 256, with the operand contract, the roundings and the k order of gemm.hip (the
-// same bits as its other tiles).
+// tiles of 128 x 128, 128 x 192 or 128 x 256, with the operand contract and the roundings of gemm.hip. Every sum is one
+// fp32 chain in k order: the bits of gemm.hip's one-chain tiles (configs 0-7, 16, 18, 23), not those of its two k groups
+// (two chains, joined at the end), which configs 19 and 27 were. Error against 64 bits of 794 x 2048 x 8192 in two splits:
+// 2.7e-7 with two chains, 4.0e-7 with one; rounded to bf16 1.65936e-3 either way.
 //
 // A few hundred rows give about one tile per CU, so a tile's time is the call's. 4 waves (2 x 2, 64 x (BN / 2) each), one
 // per SIMD, and what the 8-wave tiles that this replaced left idle between the barriers of a step is filled by writing the
@@ -8,16 +10,17 @@
 // registers of their own, so the MFMAs run across the barrier; the barrier sits in the middle of the step, behind the
 // step's last LDS read, and its slot is refilled right behind it, one load per MFMA. Loads go through buffer resources
 // (rows past the edge and steps past the end read zeros: the ring's counts hold without branches).
-// What bounds it (128 x 128, K-step of 64, ns): MFMAs alone 213, with the LDS reads 253, the loads alone 298 for one
-// workgroup and 380 with 200 of them (17 TB/s out of the L2s), everything together 390-430; the 8-wave tile before 480.
+// What bounds it (128 x 128, K-step of 64, ns, copies for timing with parts taken out): MFMAs alone 213, with the LDS reads
+// 253, the loads alone 298 for one workgroup and 380 with 200 of them (200 x 32 KB: 17 TB/s out of the L2s), everything
+// together 390-430; the 8-wave tile before 480.
 // Tried without gain: a ring of 3 or of 5 slots, lines of the next steps touched ahead (the L2 is not waited for, its rate
 // is the limit). The rest of a call is 4 us that do not depend on K: launch, first load, write-out.
-// Measured (us, cold weights, the best tile before -> this one):
-//   794 x 6144 x 2048  29.6 -> 24.7 (128 x 192; MFMAs alone 10.2)
-//   794 x 8192 x 2048, GELU  37.8 -> 33.3 (128 x 256)
-//   729 x 4304 x 1152, GELU  16.8 -> 15.4 (128 x 128)
-//   729 x 1152 x 592  9.4 -> 7.9;  1280 x 2304 x 768  11.6 -> 9.4;  730 x 6144 x 2048  29.7 -> 27.0
-// Where the grid has several tiles per CU the persistent 256-row tiles are better (9477 x 3456 x 1152: 73 against 91).
+// Measured (us, cold weights, one box, the best tile before -> this one):
+//   794 x 6144 x 2048  31.7 -> 27.9 (128 x 192; MFMAs alone 10.2)
+//   794 x 8192 x 2048, GELU  41.3 -> 35.8 (128 x 256)
+//   729 x 4304 x 1152, GELU  16.6 -> 14.3 (128 x 128)
+//   729 x 1152 x 592  9.4 -> 8.3;  1280 x 2304 x 768  12.2 -> 10.4;  730 x 6144 x 2048  29.2 -> 27.1
+// Where the grid has several tiles per CU the persistent 256-row tiles are better (9477 x 3456 x 1152: 75 against 100).
 #include "gemm_mid.h"
 
 #include "gemm_out.h"
